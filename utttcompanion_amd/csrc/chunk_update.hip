@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <mutex>
 
+#include "readout_mm.h"
 #include "update_ln.h"
 #include "uttt_device.h"
 #include "uttt_host.h"
@@ -67,9 +68,9 @@ struct FwdArgs {
 // ---------------------------------------------------------------------------
 // 1. U, G, H for one (F tile, row, path, token block)
 // ---------------------------------------------------------------------------
-template <typename T, typename WT, int KTL = KT>
+template <typename T, typename WT>
 __global__ void __launch_bounds__(kThreads) k_up_gate(const FwdArgs a) {
-  constexpr int LD = KTL + Mma<T>::kPad;
+  constexpr int LD = lds_ld<T>();
   __shared__ __align__(16) T xs[64 * LD];
   __shared__ __align__(16) T us[64 * LD];
   __shared__ __align__(16) T gs[64 * LD];
@@ -81,7 +82,7 @@ __global__ void __launch_bounds__(kThreads) k_up_gate(const FwdArgs a) {
   const T* x = key_block ? static_cast<const T*>(a.kx) + (int64_t)b * a.kx_rs
                          : static_cast<const T*>(a.x[path]) + (int64_t)b * a.x_rs[path] + (int64_t)t0 * a.D;
   // threads [0, U) stage W_up, [U, 2U) W_gate (U units of 8 rows x one 16-byte chunk)
-  constexpr int U = ColStage<WT, KTL>::kUnits;
+  constexpr int U = ColStage<WT, KT>::kUnits;
   static_assert(2 * U <= kThreads, "W_up and W_gate stage in separate halves of the workgroup");
   const bool up_half = threadIdx.x < U;
   const WT* wsrc = static_cast<const WT*>(up_half ? a.wu[path] : a.wg[path]) + (int64_t)b * a.w_rs[path] + f0;
@@ -89,23 +90,23 @@ __global__ void __launch_bounds__(kThreads) k_up_gate(const FwdArgs a) {
   const int unit = up_half ? (int)threadIdx.x : min((int)threadIdx.x - U, U);
   const int w = threadIdx.x >> 6, wr = (w >> 1) * 32, wc = (w & 1) * 32;
 
-  RowStage<T, KTL> xst;
-  ColStage<WT, KTL> wst;
+  RowStage<T, KT> xst;
+  ColStage<WT, KT> wst;
   xst.load(x, a.D, rows);
-  wst.load(wsrc, a.F, KTL, unit);
+  wst.load(wsrc, a.F, KT, unit);
   f32x16 au, ag;
   zero(au);
   zero(ag);
-  for (int d0 = 0; d0 < a.D; d0 += KTL) {
+  for (int d0 = 0; d0 < a.D; d0 += KT) {
     xst.template store<T>(xs, LD);
     wst.template store<T>(wdst, LD);
     __syncthreads();
-    if (d0 + KTL < a.D) {
-      xst.load(x + d0 + KTL, a.D, rows);
-      wst.load(wsrc + (int64_t)(d0 + KTL) * a.F, a.F, KTL, unit);
+    if (d0 + KT < a.D) {
+      xst.load(x + d0 + KT, a.D, rows);
+      wst.load(wsrc + (int64_t)(d0 + KT) * a.F, a.F, KT, unit);
     }
-    wave_mma<T, KTL>(au, xs + wr * LD, LD, us + wc * LD, LD);
-    wave_mma<T, KTL>(ag, xs + wr * LD, LD, gs + wc * LD, LD);
+    wave_mma<T, KT>(au, xs + wr * LD, LD, us + wc * LD, LD);
+    wave_mma<T, KT>(ag, xs + wr * LD, LD, gs + wc * LD, LD);
     __syncthreads();
   }
 
@@ -266,38 +267,38 @@ __global__ void __launch_bounds__(KEYS ? 512 : 256) k_up_gate_lds(const FwdArgs 
 // ---------------------------------------------------------------------------
 // 2. Z partial = H[:, split] W_down[split, D tile]
 // ---------------------------------------------------------------------------
-template <typename T, typename WT, int KTL = KT>
+template <typename T, typename WT>
 __global__ void __launch_bounds__(kThreads) k_down_partial(const FwdArgs a) {
-  constexpr int LD = KTL + Mma<T>::kPad;
+  constexpr int LD = lds_ld<T>();
   __shared__ __align__(16) T hs[64 * LD];
   __shared__ __align__(16) T ws[64 * LD];
   const int dt = blockIdx.x, split = blockIdx.y;
   const int b = blockIdx.z % a.B, pt = blockIdx.z / a.B;
   const int path = pt / a.ntb, tb = pt - path * a.ntb;
   const int d0 = dt * 64, t0 = tb * 64;
-  const int nK = a.F / KTL;  // F ranges in whole K tiles
-  const int f_begin = (nK * split / a.nsplit) * KTL, f_end = (nK * (split + 1) / a.nsplit) * KTL;
+  const int nK = a.F / KT;  // F ranges in whole K tiles
+  const int f_begin = (nK * split / a.nsplit) * KT, f_end = (nK * (split + 1) / a.nsplit) * KT;
   const T* h = static_cast<const T*>(a.h[path]) + ((int64_t)b * a.tok_pad + t0) * a.F;
   const WT* wd = static_cast<const WT*>(a.wd[path]) + (int64_t)b * a.w_rs[path] + d0;
   const int w = threadIdx.x >> 6, wr = (w >> 1) * 32, wc = (w & 1) * 32;
 
-  RowStage<T, KTL> hst;
-  ColStage<WT, KTL> wst;  // W_down rows f, columns d -> [d][f]
+  RowStage<T, KT> hst;
+  ColStage<WT, KT> wst;  // W_down rows f, columns d -> [d][f]
   f32x16 acc;
   zero(acc);
   if (f_begin < f_end) {
     hst.load(h + f_begin, a.F, 64);
-    wst.load(wd + (int64_t)f_begin * a.D, a.D, KTL, threadIdx.x);
+    wst.load(wd + (int64_t)f_begin * a.D, a.D, KT, threadIdx.x);
   }
-  for (int f0 = f_begin; f0 < f_end; f0 += KTL) {
+  for (int f0 = f_begin; f0 < f_end; f0 += KT) {
     hst.template store<T>(hs, LD);
     wst.template store<T>(ws, LD);
     __syncthreads();
-    if (f0 + KTL < f_end) {
-      hst.load(h + f0 + KTL, a.F, 64);
-      wst.load(wd + (int64_t)(f0 + KTL) * a.D, a.D, KTL, threadIdx.x);
+    if (f0 + KT < f_end) {
+      hst.load(h + f0 + KT, a.F, 64);
+      wst.load(wd + (int64_t)(f0 + KT) * a.D, a.D, KT, threadIdx.x);
     }
-    wave_mma<T, KTL>(acc, hs + wr * LD, LD, ws + wc * LD, LD);
+    wave_mma<T, KT>(acc, hs + wr * LD, LD, ws + wc * LD, LD);
     __syncthreads();
   }
   float* zp = a.zp + ((((int64_t)path * a.nsplit + split) * a.B + b) * a.tok_pad + t0) * a.D + d0;
@@ -323,7 +324,7 @@ __global__ void __launch_bounds__(kThreads) k_down_partial_lds(const FwdArgs a, 
   const int b = rt.b % a.B, pt = rt.b / a.B;
   const int path = pt / a.ntb, tb = pt - path * a.ntb;
   const int d0 = dt * 64, t0 = tb * 64;
-  const int nK = a.F / kb;  // F ranges in whole blocks of kb, as k_down_partial<.., kb>
+  const int nK = a.F / kb;  // F ranges in whole blocks of kb
   const int f_begin = (nK * split / a.nsplit) * kb, f_end = (nK * (split + 1) / a.nsplit) * kb;
   const int nsteps = (f_end - f_begin) / 64;
   const bf16* h = static_cast<const bf16*>(a.h[path]) + ((int64_t)b * a.tok_pad + t0) * a.F + f_begin;
@@ -1119,7 +1120,11 @@ struct ReadoutLayout {
 static ReadoutLayout readout_layout(int64_t B, int64_t T, int64_t D, int64_t F, int32_t dtype) {
   ReadoutLayout L;
   L.ntb = (int)((T + 63) / 64);
-  L.nsplit = pick_nsplit((D / 64) * B * L.ntb, F / 64);
+  // long bf16 blocks: the products of readout_mm.hip, whose split depends on the weights' type;
+  // the workspace holds either
+  L.nsplit = L.ntb > 1 && dtype == UTTT_DTYPE_BF16
+                 ? std::max(readout_mm_splits(B, T, D, F, false), readout_mm_splits(B, T, D, F, true))
+                 : pick_nsplit((D / 64) * B * L.ntb, F / 64);
   // one token: room for the GEMV's F-block partials too
   const int64_t zsplits = T == 1 ? std::max<int64_t>(L.nsplit, F / gemv_fb(F)) : L.nsplit;
   size_t off = 0;
@@ -1172,41 +1177,42 @@ static void launch_readout(const uttt_readout_args& a, char* ws, const ReadoutLa
       return;
     }
   }
-  // bf16 weights: K tiles of 128 halve the staged steps of these latency-bound loops where the
-  // shape allows.  The key block (when asked for) is one more z block: it runs beside the token
-  // blocks of the same F tile and row, on the same XCD, so its weight tiles come from that L2.
-  constexpr bool wide = sizeof(WT) == 2;
-  const dim3 ug_grid(F / 64, B, L.ntb + (a.keys != nullptr ? 1 : 0));
-  if constexpr (sizeof(T) == 2 && sizeof(WT) == 2) {
-    if (L.ntb == 1) {  // one token block: the LDS-ring kernel
-      if (F % 128 == 0) {
-        if (a.keys != nullptr)
-          hipLaunchKernelGGL((k_up_gate_lds<true, 2>), dim3(row_tile_blocks(B, F / 128)), dim3(512), 0, st, f);
-        else
-          hipLaunchKernelGGL((k_up_gate_lds<false, 2>), dim3(row_tile_blocks(B, F / 128)), dim3(256), 0, st, f);
-      } else if (a.keys != nullptr) {
-        hipLaunchKernelGGL((k_up_gate_lds<true, 1>), dim3(row_tile_blocks(B, F / 64)), dim3(512), 0, st, f);
-      } else {
-        hipLaunchKernelGGL((k_up_gate_lds<false, 1>), dim3(row_tile_blocks(B, F / 64)), dim3(256), 0, st, f);
-      }
-    } else if (D % 128 == 0) {
-      hipLaunchKernelGGL((k_up_gate<T, WT, 128>), ug_grid, blk, 0, st, f);
-    } else {
-      hipLaunchKernelGGL((k_up_gate<T, WT>), ug_grid, blk, 0, st, f);
+  if constexpr (sizeof(T) == 2) {
+    if (L.ntb > 1) {
+      ReadoutMmArgs m{};
+      m.B = B; m.T = f.ntok; m.D = D; m.F = F; m.tok_pad = f.tok_pad;
+      m.x = a.x; m.x_rs = a.x_row_stride;
+      m.w_up = a.w_up; m.w_gate = a.w_gate; m.w_down = a.w_down; m.w_rs = a.w_row_stride;
+      m.w_fp32 = sizeof(WT) == 4;
+      m.h = f.h[0]; m.zp = f.zp;
+      launch_readout_mm(m, st);
+      LnOutArgs o{};
+      o.B = B; o.ntok = (int)a.tokens; o.D = D; o.tok_pad = f.tok_pad; o.eps = a.eps;
+      o.nsplit = readout_mm_splits(B, a.tokens, D, F, m.w_fp32);
+      o.zp = f.zp; o.x = a.x; o.x_rs = a.x_row_stride; o.ln_w = a.ln_weight; o.ln_b = a.ln_bias;
+      o.out = a.out; o.out_rs = a.out_row_stride;
+      launch_ln_readout<T>(dim3((unsigned)a.tokens, B), st, o);
+      return;
     }
-  } else if (wide && D % 128 == 0) {
-    hipLaunchKernelGGL((k_up_gate<T, WT, wide ? 128 : KT>), ug_grid, blk, 0, st, f);
-  } else {
-    hipLaunchKernelGGL((k_up_gate<T, WT>), ug_grid, blk, 0, st, f);
   }
-  const dim3 dp_grid(D / 64, L.nsplit, L.ntb * B);
-  if constexpr (sizeof(T) == 2 && sizeof(WT) == 2)
-    hipLaunchKernelGGL(k_down_partial_lds, dim3(row_tile_blocks(L.ntb * B, (D / 64) * L.nsplit)), blk, 0, st, f,
+  if constexpr (sizeof(T) == 2 && sizeof(WT) == 2) {  // one token block: the LDS-ring kernels
+    const bool keys = a.keys != nullptr;
+    if (F % 128 == 0 && keys)
+      hipLaunchKernelGGL((k_up_gate_lds<true, 2>), dim3(row_tile_blocks(B, F / 128)), dim3(512), 0, st, f);
+    else if (F % 128 == 0)
+      hipLaunchKernelGGL((k_up_gate_lds<false, 2>), dim3(row_tile_blocks(B, F / 128)), dim3(256), 0, st, f);
+    else if (keys)
+      hipLaunchKernelGGL((k_up_gate_lds<true, 1>), dim3(row_tile_blocks(B, F / 64)), dim3(512), 0, st, f);
+    else
+      hipLaunchKernelGGL((k_up_gate_lds<false, 1>), dim3(row_tile_blocks(B, F / 64)), dim3(256), 0, st, f);
+    hipLaunchKernelGGL(k_down_partial_lds, dim3(row_tile_blocks(B, (D / 64) * L.nsplit)), blk, 0, st, f,
                        F % 128 == 0 ? 128 : KT);
-  else if (wide && F % 128 == 0)
-    hipLaunchKernelGGL((k_down_partial<T, WT, wide ? 128 : KT>), dp_grid, blk, 0, st, f);
-  else
-    hipLaunchKernelGGL((k_down_partial<T, WT>), dp_grid, blk, 0, st, f);
+  } else {
+    // the key block (when asked for) is one more z block: it runs beside the token block of the
+    // same F tile and row, on the same XCD, so its weight tiles come from that L2
+    hipLaunchKernelGGL((k_up_gate<T, WT>), dim3(F / 64, B, L.ntb + (a.keys != nullptr ? 1 : 0)), blk, 0, st, f);
+    hipLaunchKernelGGL((k_down_partial<T, WT>), dim3(D / 64, L.nsplit, L.ntb * B), blk, 0, st, f);
+  }
   LnOutArgs o{};
   o.B = B; o.ntok = (int)a.tokens; o.D = D; o.nsplit = L.nsplit; o.tok_pad = f.tok_pad; o.eps = a.eps;
   o.zp = f.zp; o.x = a.x; o.x_rs = a.x_row_stride; o.ln_w = a.ln_weight; o.ln_b = a.ln_bias;
