@@ -1,12 +1,16 @@
 // Sliding-window GQA attention for the uTTT blocks on gfx950 (MI355X):
 //   * k_rope_append  -- RoPE on q (in place) and k, append rotated k and v to a KV buffer
-//   * k_swa_prefill  -- flash-style attention: 64 queries per workgroup, 64-key LDS tiles,
-//                       only the key tiles that intersect the window are visited
+//   * k_swa_prefill  -- flash-style attention for fp32 operands: 64 queries per workgroup, 64-key
+//                       LDS tiles, only the key tiles that intersect the window are visited
+//                       (bf16 operands: swa_prefill.hip)
 //   * k_swa_decode   -- one token per request over a ring-buffer KV cache
 // Visibility rule (reference model/uttt_layer.py:1028-1037): query at absolute key index p
 // sees key j iff 0 <= p - j < window; kv head = h / (n_heads / n_kv_heads).
 #include <math.h>
 
+#include <algorithm>
+
+#include "swa_prefill.h"
 #include "uttt_device.h"
 #include "uttt_host.h"
 
@@ -971,9 +975,13 @@ __global__ void __launch_bounds__(kThreads) k_swa_decode_combine(const uttt_swa_
 template <typename T, int HD>
 static void launch_prefill(const uttt_swa_prefill_args& a, const PrefillPlan& p, hipStream_t st) {
   float* part = static_cast<float*>(a.workspace);
-  const dim3 grid((unsigned)row_tile_blocks((int)(a.batch * a.n_kv_heads), p.nqt * (int)(a.n_heads / a.n_kv_heads) * p.nsplit));
-  hipLaunchKernelGGL((k_swa_prefill<T, HD>), grid, dim3(kThreads), 0, st, a, part, p.nsplit, p.tiles_per_split,
-                     p.q_pad, p.nqt);
+  if constexpr (sizeof(T) == 2) {
+    launch_swa_prefill_mm(a, part, p.q_pad, st);
+  } else {
+    const dim3 grid((unsigned)row_tile_blocks((int)(a.batch * a.n_kv_heads), p.nqt * (int)(a.n_heads / a.n_kv_heads) * p.nsplit));
+    hipLaunchKernelGGL((k_swa_prefill<T, HD>), grid, dim3(kThreads), 0, st, a, part, p.nsplit, p.tiles_per_split,
+                       p.q_pad, p.nqt);
+  }
   if (p.nsplit > 1)
     hipLaunchKernelGGL((k_swa_prefill_combine<T, HD>),
                        dim3((unsigned)((int64_t)p.q_pad * HD / (kThreads * kCombineEpt)), (unsigned)a.n_heads,
@@ -1036,9 +1044,11 @@ extern "C" int uttt_rope_kv_append(const uttt_rope_append_args* a, uttt_stream_t
 extern "C" size_t uttt_swa_prefill_workspace(int64_t batch, int64_t n_heads, int64_t q_len, int64_t kv_len,
                                              int64_t head_dim, int64_t window) {
   if (batch < 1 || n_heads < 1 || q_len < 1 || kv_len < 1 || window < 1 || head_dim < 1) return 0;
+  // the query does not name the type or the kv heads: room for either type's splits
   const PrefillPlan p = prefill_plan(batch, n_heads, q_len, kv_len, window);
-  if (p.nsplit == 1) return 16;
-  return sizeof(float) * (size_t)p.nsplit * (size_t)batch * (size_t)n_heads * (size_t)p.q_pad * (size_t)(head_dim + 2);
+  const int nsplit = std::max(p.nsplit, swa_prefill_mm_max_splits(batch, n_heads, q_len, kv_len, window));
+  if (nsplit == 1) return 16;
+  return sizeof(float) * (size_t)nsplit * (size_t)batch * (size_t)n_heads * (size_t)p.q_pad * (size_t)(head_dim + 2);
 }
 
 extern "C" int uttt_swa_prefill(const uttt_swa_prefill_args* a, uttt_stream_t stream) {
@@ -1061,7 +1071,8 @@ extern "C" int uttt_swa_prefill(const uttt_swa_prefill_args* a, uttt_stream_t st
   UTTT_REQUIRE(a->k_stride_t >= a->head_dim && a->v_stride_t >= a->head_dim &&
                    a->k_stride_t * 64 * 4 <= 0x7fffffffLL && a->v_stride_t * 64 * 4 <= 0x7fffffffLL,
                "k/v token strides must cover a row and fit a 64-row buffer range");
-  const PrefillPlan p = prefill_plan(a->batch, a->n_heads, a->q_len, a->kv_len, a->window);
+  PrefillPlan p = prefill_plan(a->batch, a->n_heads, a->q_len, a->kv_len, a->window);
+  if (a->act_dtype == UTTT_DTYPE_BF16) p.nsplit = swa_prefill_mm_splits(*a);
   UTTT_REQUIRE(a->batch * p.nsplit <= 65535 && a->batch * a->n_heads * p.nqt * p.nsplit + 8LL * a->n_heads <= 0x7fffffffLL,
                "batch too large for the attention grid");
   UTTT_REQUIRE(p.nsplit == 1 || (a->workspace != nullptr &&
