@@ -1,0 +1,75 @@
+"""The bf16 chunk update against float64 at the edges of its tiles: one token to several token
+blocks, the smallest and ragged widths, reads through the cursor's own weights (one matrix of K and Q
+rows), through other weights and through shared ones, masks, in place and into unaligned outputs."""
+import pytest
+import torch
+
+from oracle import uttt_math as om
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # rows, tokens, d_model, d_ff, read, masked, clip
+    (1, 1, 64, 64, "own", False, 1.0),
+    (3, 63, 128, 192, "own", True, 1.0),
+    (2, 64, 192, 64, "other", False, 0.01),   # the clip is active
+    (1, 64, 576, 1088, "own", False, 0.0),    # no clip
+    (5, 65, 128, 128, "other", True, 0.01),   # two token blocks, rows not a power of two
+    (2, 129, 64, 320, "shared", False, 0.01), # three token blocks
+    (1, 300, 256, 192, "own", True, 0.01),    # five
+    (8, 37, 320, 256, "shared", True, 1.0),
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("out", ["new", "in_place", "unaligned"])
+def test_update_matches_float64(case, out):
+    from utttcompanion_amd import kernels as K
+    b, c, d, f, read, masked, clip = case
+    print(f"update {case} {out}", flush=True)
+    g = torch.Generator().manual_seed(sum(case[:4]))
+    unit = lambda: torch.nn.functional.rms_norm(torch.randn(b, c, d, generator=g), (d,)).bfloat16()
+    q, k, v = unit(), unit(), unit()
+    eta = (0.015 * torch.rand(b, c, 1, generator=g)).bfloat16()
+    alpha = (0.005 * torch.rand(b, c, 1, generator=g)).bfloat16()
+    weights = lambda n: [torch.randn(n, d, f, generator=g) / d ** 0.5, torch.randn(n, d, f, generator=g) / d ** 0.5,
+                         torch.randn(n, f, d, generator=g) * 0.1 / f ** 0.5]
+    w = weights(b)
+    s = [1e-4 * t for t in weights(b)]
+    rd = None if read == "own" else weights(1 if read == "shared" else b)
+    ln = [1 + 0.1 * torch.randn(d, generator=g), 0.1 * torch.randn(d, generator=g)]
+    mask = None
+    if masked:
+        mask = (torch.arange(c)[None] < torch.randint(0, c + 1, (b, 1), generator=g)).float()
+        mask[0] = 0.0  # a row without tokens
+    dev = lambda ts: [t.cuda() for t in ts]
+    state = dev(w) + dev(s)
+    outs = None
+    if out == "in_place":
+        outs = state
+    elif out == "unaligned":  # one float past an aligned address
+        outs = [torch.empty(t.numel() + 1, device="cuda")[1:].view(t.shape) for t in state]
+    res = K.chunk_update(*dev([q, k, v, eta, alpha]), *state, *dev(ln), None if mask is None else mask.cuda(), 0.9,
+                         clip, True, 1e-5, *(dev(rd) if rd else (None,) * 3), out_state=outs)
+    rd64 = None if rd is None else [t.bfloat16().double().expand(b, -1, -1) for t in rd]
+    w16 = [t.bfloat16().double() for t in w]  # the operands of the matrix units
+    ref = om.fused_chunk_ttt_step(q.double(), k.double(), v.double(), eta.double(), alpha.double(), *w16,
+                                  *(t.double() for t in s), *(t.double() for t in ln),
+                                  None if mask is None else mask.double(), 0.9, clip, True, 1e-5,
+                                  *(rd64 or w16))
+    decay = 1.0 - (alpha[..., 0].double().mean(1) if mask is None else
+                   (alpha[..., 0].double() * mask.double()).sum(1) / mask.double().sum(1).clamp_min(1)).view(-1, 1, 1)
+    live = torch.ones(b, 1, 1) if mask is None else mask.any(1).view(-1, 1, 1).float()
+    # H, dZ, dU and dG are rounded once (2^-9 relative at most): a gradient sums products of two of
+    # them or of one and K, so its norm is off by at most about 2 * 2^-9; doubled for the clip factor
+    for i in range(3):
+        step = ref[4 + i] - 0.9 * s[i].double() * live - s[i].double() * (1 - live)
+        got = res[4 + i].double().cpu() - 0.9 * s[i].double() * live - s[i].double() * (1 - live)
+        floor = 1e-6 * float(s[i].double().norm())  # the fp32 momentum's own rounding
+        assert float((got - step).norm()) <= 2.0 ** -7 * float(step.norm()) + floor, ("s", i)
+        new_w = torch.where(live.bool(), decay * w[i].double() + res[4 + i].double().cpu(), w[i].double())
+        assert float((res[1 + i].double().cpu() - new_w).abs().max()) <= 4 * 2.0 ** -24 * float(new_w.abs().max()), ("w", i)
+    # the readout as in the frozen one: output rounding, and H's through the LayerNorm
+    bound = 2.0 ** -8 * ref[0].abs() + 7 * 2.0 ** -9 / 3 ** 0.5 * 2.0
+    assert bool(((res[0].double().cpu() - ref[0]).abs() <= bound).all())
+    assert abs(float(res[7]) - float(ref[7])) <= 2.0 ** -8 * abs(float(ref[7]))

@@ -11,20 +11,22 @@
 //   readout O = Q + LN((SiLU(Q R_gate) * Q R_up) R_down)   (R = read snapshot)
 // (reference: model/uttt_layer.py:279-534)
 //
-// Kernel sequence for one chunk (all rows in each launch):
-//   1. k_up_gate      U/G/H for the K path (cursor W) and the Q path (read W), per F tile
-//   2. k_down_partial Z partial sums over F splits, per D tile
-//   3. k_ln_grad      LN + loss + dZ per token (K path)
-//   4. k_ln_readout   LN + residual readout per token (Q path)
-//   5. k_backward     dH, dU, dG per F tile + the per-row squared gradient norm partial
-//   6. k_apply        recompute each gradient tile from the small activations and apply
-//                     clip / momentum / decay / inactive-row select to W and S in one pass
-// Steps 1, 2 and 4 alone are the frozen readout.
+// Kernel sequence for one chunk (all rows in each launch), fp32 activations / bf16 activations:
+//   1. k_up_gate / readout_mm.hip       U/G/H for the K path (cursor W) and the Q path (read W)
+//   2. k_down_partial / readout_mm.hip  Z partial sums over F splits, per D tile
+//   3. k_ln_both                        LN + loss + dZ per token (K path), LN + residual readout
+//                                       per token (Q path)
+//   4. k_backward / update_mm.hip       dH, dU, dG per F tile + the squared gradient norm partials
+//   5. k_apply / update_mm.hip          recompute each gradient tile from the small activations and
+//                                       apply clip / momentum / decay / inactive-row select to W
+//                                       and S in one pass (bf16: k_row_scalars first)
+// Steps 1, 2 and the readout half of 3 alone are the frozen readout.
 #include <algorithm>
 #include <mutex>
 
 #include "readout_mm.h"
 #include "update_ln.h"
+#include "update_mm.h"
 #include "uttt_device.h"
 #include "uttt_host.h"
 
@@ -502,6 +504,32 @@ static void launch_ln_readout(dim3 grid, hipStream_t st, const LnOutArgs& o) {
     hipLaunchKernelGGL((k_ln_readout<T, 16>), grid, dim3(kThreads), 0, st, o);
 }
 
+// The LayerNorm gradient of the K path (z 0) and the readout of the Q path (z 1) in one launch:
+// both are a few microseconds of latency, and neither reads what the other writes.
+template <typename T, int KPER>
+__global__ void __launch_bounds__(kThreads) k_ln_both(const LnGradArgs g, const LnOutArgs a) {
+  __shared__ float red[4], red2[8];
+  const int t = blockIdx.x, b = blockIdx.y;
+  if (blockIdx.z == 0) {
+    ln_grad_row<T, KPER>(g, t, b, red, red2);
+    return;
+  }
+  if (t >= a.ntok) return;
+  ln_readout_row<T, KPER>(a.zp + ((int64_t)b * a.tok_pad + t) * a.D, (int64_t)a.B * a.tok_pad * a.D, a.nsplit, a.D,
+                          a.eps, a.ln_w, a.ln_b, static_cast<const T*>(a.x) + (int64_t)b * a.x_rs + (int64_t)t * a.D,
+                          static_cast<T*>(a.out) + (int64_t)b * a.out_rs + (int64_t)t * a.D, red);
+}
+
+template <typename T>
+static void launch_ln_both(dim3 grid, hipStream_t st, const LnGradArgs& g, const LnOutArgs& o) {
+  if (o.D <= 4 * kThreads)
+    hipLaunchKernelGGL((k_ln_both<T, 4>), grid, dim3(kThreads), 0, st, g, o);
+  else if (o.D <= 8 * kThreads)
+    hipLaunchKernelGGL((k_ln_both<T, 8>), grid, dim3(kThreads), 0, st, g, o);
+  else
+    hipLaunchKernelGGL((k_ln_both<T, 16>), grid, dim3(kThreads), 0, st, g, o);
+}
+
 // ---------------------------------------------------------------------------
 // 5. dH = dZ W_down^T per F tile; dU, dG; squared-norm partial of all three gradients
 // ---------------------------------------------------------------------------
@@ -635,7 +663,7 @@ struct ApplyArgs {
   float min_row_surprise;  // > 0: rows whose chunk surprise is below it keep W and S
 };
 
-// The last wave of an apply workgroup derives its row's clip factor, decay and active flag (and,
+// fp32 path: the last wave of an apply workgroup derives its row's clip factor, decay and active flag (and,
 // in the first workgroups, the row's loss sums and the batch-global surprise).
 template <typename T>
 __device__ __forceinline__ void apply_row_scalars(const ApplyArgs& a, int b, float* row_scalar) {
@@ -696,6 +724,48 @@ __device__ __forceinline__ void apply_row_scalars(const ApplyArgs& a, int b, flo
       if (lane == 0) *a.surprise = a.mask != nullptr ? num / fmaxf(den, 1.f) : num / den;
     }
   }
+}
+
+// The same scalars once per row (bf16 path): out (B, 4) = clip factor, decay, active flag.  A chunk
+// of several token blocks has a norm partial per gradient tile (2112 at d 1024, F 2816), too many
+// for every workgroup of the apply to sum: that took most of its 147 us at 2 rows of 128 tokens.
+template <typename T>
+__global__ void __launch_bounds__(kThreads) k_row_scalars(const ApplyArgs a, float* out) {
+  __shared__ float red[20];
+  const int b = blockIdx.x;
+  float v[5] = {0.f, 0.f, 0.f, 0.f, 0.f};  // squared norm, alpha sum, valid tokens, any valid, loss sum
+  if (a.max_norm > 0.f)
+    for (int i = threadIdx.x; i < a.n_norm; i += kThreads) v[0] += a.nrm[(int64_t)b * a.n_norm + i];
+  const T* al = static_cast<const T*>(a.alpha) + (int64_t)b * a.alpha_rs;
+  for (int t = threadIdx.x; t < a.C; t += kThreads) {
+    const float mt = a.mask != nullptr ? a.mask[(int64_t)b * a.mask_rs + t] : 1.f;
+    v[1] += a.mask != nullptr ? to_f32(al[t]) * mt : to_f32(al[t]);
+    v[2] += mt;
+    v[3] += mt != 0.f ? 1.f : 0.f;
+    v[4] += a.loss[(int64_t)b * a.tok_pad + t];
+  }
+  block_sums<5>(v, red);
+  if (threadIdx.x == 0) {
+    const float n = a.mask != nullptr ? fmaxf(v[2], 1.f) : (float)a.C;
+    const bool gated_off = a.min_row_surprise > 0.f && v[4] / fmaxf(n, 1.f) < a.min_row_surprise;
+    out[4 * b] = a.max_norm > 0.f ? fminf(a.max_norm * (1.0f / sqrtf(v[0] + 1e-8f)), 1.0f) : 1.0f;
+    out[4 * b + 1] = 1.0f - v[1] / n;
+    out[4 * b + 2] = ((a.mask == nullptr || v[3] > 0.f) && !gated_off) ? 1.f : 0.f;
+    if (a.row_loss != nullptr) {
+      a.row_loss[2 * b] = v[4];
+      a.row_loss[2 * b + 1] = v[2];
+    }
+  }
+  if (b != 0) return;
+  // batch-global surprise: sum of masked token losses over all rows / valid tokens
+  float s[2] = {0.f, 0.f};
+  for (int i = threadIdx.x; i < a.B * a.tok_pad; i += kThreads) {
+    const int bb = i / a.tok_pad, t = i - bb * a.tok_pad;
+    s[0] += a.loss[i];
+    if (t < a.C) s[1] += a.mask != nullptr ? a.mask[(int64_t)bb * a.mask_rs + t] : 1.f;
+  }
+  block_sums<2>(s, red);
+  if (threadIdx.x == 0) *a.surprise = a.mask != nullptr ? s[0] / fmaxf(s[1], 1.f) : s[0] / s[1];
 }
 
 // NORM: instead of applying, write the tile's squared Frobenius norm to nrm (one partial per tile):
@@ -861,25 +931,41 @@ static void launch_update(const uttt_chunk_update_args& a, char* ws, const Updat
   const dim3 blk(kThreads);
   auto want = [&](int phase) { return first_phase <= phase && phase <= last_phase; };
 
-  if (want(0)) hipLaunchKernelGGL((k_up_gate<T, float>), dim3(F / 64, B, 2 * ntb), blk, 0, st, f);
-  if (want(1)) hipLaunchKernelGGL((k_down_partial<T, float>), dim3(D / 64, L.nsplit, 2 * ntb * B), blk, 0, st, f);
+  // bf16: the K and Q rows as one matrix where both read the same weights
+  const bool joint = a.r_up == a.w_up && a.r_gate == a.w_gate && a.r_down == a.w_down &&
+                     (a.r_row_stride == (int64_t)D * F || B == 1);
+  int nsplit = L.nsplit;
+  if constexpr (sizeof(T) == 2) {
+    UpdateMmArgs m{};
+    m.B = B; m.T = C; m.D = D; m.F = F; m.tok_pad = TP;
+    for (int s = 0; s < 2; ++s) {
+      m.x[s] = f.x[s]; m.x_rs[s] = f.x_rs[s]; m.h[s] = f.h[s]; m.w_rs[s] = f.w_rs[s];
+      m.w_up[s] = static_cast<const float*>(f.wu[s]);
+      m.w_gate[s] = static_cast<const float*>(f.wg[s]);
+      m.w_down[s] = static_cast<const float*>(f.wd[s]);
+    }
+    m.u_store = f.u_store; m.g_store = f.g_store; m.zp = f.zp; m.splits = L.nsplit;
+    nsplit = update_mm_splits(B, C, D, F, joint, L.nsplit);
+    if (want(0)) launch_update_up(m, joint, st);
+    if (want(1)) launch_update_down(m, joint, st);
+  } else {
+    if (want(0)) hipLaunchKernelGGL((k_up_gate<T, float>), dim3(F / 64, B, 2 * ntb), blk, 0, st, f);
+    if (want(1)) hipLaunchKernelGGL((k_down_partial<T, float>), dim3(D / 64, L.nsplit, 2 * ntb * B), blk, 0, st, f);
+  }
 
   LnGradArgs g{};
-  g.B = B; g.C = C; g.D = D; g.nsplit = L.nsplit; g.tok_pad = TP; g.normalize = a.normalize_by_dim;
+  g.B = B; g.C = C; g.D = D; g.nsplit = nsplit; g.tok_pad = TP; g.normalize = a.normalize_by_dim;
   g.eps = a.eps; g.zp = f.zp;
   g.k = a.k; g.k_rs = a.k_row_stride; g.v = a.v; g.v_rs = a.v_row_stride;
   g.eta = a.eta; g.eta_rs = a.eta_row_stride; g.mask = a.token_mask; g.mask_rs = a.mask_row_stride;
   g.ln_w = a.ln_weight; g.ln_b = a.ln_bias;
   g.dz = ws + L.dz; g.loss = reinterpret_cast<float*>(ws + L.loss);
   LnOutArgs o{};
-  o.B = B; o.ntok = C; o.D = D; o.nsplit = L.nsplit; o.tok_pad = TP; o.eps = a.eps;
-  o.zp = f.zp + (size_t)L.nsplit * B * TP * D;
+  o.B = B; o.ntok = C; o.D = D; o.nsplit = nsplit; o.tok_pad = TP; o.eps = a.eps;
+  o.zp = f.zp + (size_t)nsplit * B * TP * D;
   o.x = a.q; o.x_rs = a.q_row_stride; o.ln_w = a.ln_weight; o.ln_b = a.ln_bias;
   o.out = a.out; o.out_rs = a.out_row_stride;
-  if (want(2)) {
-    launch_ln_grad<T>(dim3(TP, B), st, g);
-    launch_ln_readout<T>(dim3(C, B), st, o);
-  }
+  if (want(2)) launch_ln_both<T>(dim3(TP, B, 2), st, g, o);
 
   BwdArgs bw{};
   bw.B = B; bw.C = C; bw.D = D; bw.F = F; bw.ntb = ntb; bw.tok_pad = TP;
@@ -899,13 +985,36 @@ static void launch_update(const uttt_chunk_update_args& a, char* ws, const Updat
   ap.surprise = a.surprise;
   ap.row_loss = a.row_loss;
   ap.min_row_surprise = a.min_row_surprise;
-  const dim3 tiles(3 * (D / 64) * (F / 64), B);
-  if (want(3)) {
-    hipLaunchKernelGGL(k_backward<T>, dim3(F / 64, B, ntb), blk, 0, st, bw);
-    // a chunk of several token blocks: each gradient tile's squared norm over the whole chunk
-    if (ntb > 1) hipLaunchKernelGGL((k_apply<T, true>), tiles, blk, 0, st, ap);
+  if constexpr (sizeof(T) == 2) {
+    UpdateWriteArgs u{};
+    u.B = B; u.C = C; u.D = D; u.F = F; u.ntb = ntb; u.tok_pad = TP;
+    u.k = a.k; u.k_rs = a.k_row_stride; u.h = f.h[0]; u.dz = g.dz; u.du = bw.du; u.dg = bw.dg;
+    for (int i = 0; i < 3; ++i) {
+      u.w[i] = ap.w[i]; u.s[i] = ap.s[i]; u.w_out[i] = ap.w_out[i]; u.s_out[i] = ap.s_out[i];
+    }
+    float* scalars = f.zp;  // the Z partials are consumed by then
+    u.beta = a.momentum_beta; u.nrm = bw.nrm; u.scalars = scalars;
+    if (want(3)) {
+      UpdateBackArgs k{};
+      k.B = B; k.C = C; k.D = D; k.F = F; k.ntb = ntb; k.tok_pad = TP;
+      k.k = a.k; k.k_rs = a.k_row_stride; k.w_down = a.w_down; k.u = f.u_store; k.g = f.g_store;
+      k.h = f.h[0]; k.dz = g.dz; k.du = bw.du; k.dg = bw.dg; k.nrm = bw.nrm;
+      launch_update_back(k, st);
+      // a chunk of several token blocks: each gradient tile's squared norm over the whole chunk
+      if (ntb > 1 && a.max_inner_grad_norm > 0.f) launch_update_norm(u, st);
+    }
+    if (want(4)) {
+      hipLaunchKernelGGL(k_row_scalars<T>, dim3(B), blk, 0, st, ap, scalars);
+      launch_update_write(u, st);
+    }
+  } else {
+    const dim3 tiles(3 * (D / 64) * (F / 64), B);
+    if (want(3)) {
+      hipLaunchKernelGGL(k_backward<T>, dim3(F / 64, B, ntb), blk, 0, st, bw);
+      if (ntb > 1) hipLaunchKernelGGL((k_apply<T, true>), tiles, blk, 0, st, ap);
+    }
+    if (want(4)) hipLaunchKernelGGL((k_apply<T, false>), tiles, blk, 0, st, ap);
   }
-  if (want(4)) hipLaunchKernelGGL((k_apply<T, false>), tiles, blk, 0, st, ap);
 }
 
 void launch_saved_readout(int B, int ntok, int D, int F, int nsplit, const float* h, const float* w_down,

@@ -22,6 +22,31 @@ struct ReadoutMmArgs {
   float* zp;   // fp32 (readout_mm_splits(..), B, tok_pad, D)
 };
 
+// The forward products of a chunk update (K rows through the cursor weights, Q rows through the read
+// weights): the same products with two row sets.  Where both sets read the same weights they form
+// one matrix of 2 tok_pad rows per batch row, so that a weight tile is read once for both.
+struct UpdateMmArgs {
+  int B, T, D, F;
+  int tok_pad;
+  const void* x[2];  // bf16 (B, T, D), token stride D: K, Q
+  int64_t x_rs[2];
+  const float* w_up[2];
+  const float* w_gate[2];
+  const float* w_down[2];
+  int64_t w_rs[2];
+  void* h[2];      // bf16 (B, tok_pad, F)
+  float* u_store;  // fp32 (B, tok_pad, F): K rows' products
+  float* g_store;
+  float* zp;  // fp32 (2, splits, B, tok_pad, D)
+  int splits;
+};
+
+// Splits of the update's down product, at most `most`.
+int update_mm_splits(int64_t B, int64_t T, int64_t D, int64_t F, bool joint, int most);
+
+void launch_update_up(const UpdateMmArgs& a, bool joint, hipStream_t st);
+void launch_update_down(const UpdateMmArgs& a, bool joint, hipStream_t st);
+
 // How many partials the down product leaves for the LayerNorm to sum.
 int readout_mm_splits(int64_t B, int64_t T, int64_t D, int64_t F, bool w_fp32);
 

@@ -29,17 +29,23 @@
 namespace uttt {
 namespace {
 
+// nseg row sets (segments) per batch row, rows_pad rows each (a multiple of 64, so a 64-row tile
+// lies in one segment).  joint: one matrix of nseg rows_pad rows with segment 0's weights;
+// otherwise each segment is a matrix of its own.
 struct MmArgs {
-  int B, rows, rows_pad, K, N;  // rows of A that exist, rows of the output per batch row
-  const bf16* a;                // (B, rows, K)
-  int64_t a_rs;
+  int B, nseg, joint;
+  int rows, rows_pad, K, N;  // rows of A that exist, rows of the output per batch row and segment
+  const bf16* a[2];          // (B, rows, K)
+  int64_t a_rs[2];
   int a_ld;
-  const void* w[2];  // (B | 1, K, N): the two factors of the gated product, or W_down
-  int64_t w_rs;
+  const void* w[2][2];  // per segment (B | 1, K, N): the two factors of the gated product, or W_down
+  int64_t w_rs[2];
   int splits;
   int mtiles, ntiles;
-  bf16* h;    // gated product: (B, rows_pad, N)
-  float* zp;  // down product: (splits, B, rows_pad, N)
+  bf16* h[2];  // gated product: (B, rows_pad, N)
+  float* u;    // gated product: segment 0's two factors' products, fp32 (B, rows_pad, N), or null
+  float* g;
+  float* zp;  // down product: (nseg, splits, B, rows_pad, N)
 };
 
 // LDS reads of one k piece of 16: MB A fragments (32 rows each, 4 KB apart) and 2 B fragments
@@ -109,19 +115,22 @@ __global__ void __launch_bounds__(WM* WN * 64) k_readout_mm(const MmArgs a) {
   rest /= a.mtiles;
   const int nt = rest % a.ntiles;
   rest /= a.ntiles;
-  const int split = rest % a.splits, b = rest / a.splits;
-  const int m0 = mt * MT;
+  const int split = rest % a.splits, bs = rest / a.splits;
+  const int seg0 = bs / a.B, b = bs - seg0 * a.B;  // joint: always segment 0
+  const int m0 = mt * MT, m_end = a.joint ? a.nseg * a.rows_pad : a.rows_pad;
+  // a row of the matrix -> its segment, and where that begins
+  auto seg_of = [&](int row) { return a.joint ? min(row / a.rows_pad, a.nseg - 1) : seg0; };
+  auto seg_row = [&](int seg) { return a.joint ? seg * a.rows_pad : 0; };
   const int n0 = nt * (GATED ? 32 * NS : 64 * NS);  // first column of each factor
   const int steps_all = a.K / 64;
   const int s_begin = split * steps_all / a.splits, nsteps = (split + 1) * steps_all / a.splits - s_begin;
 
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wm = w / WN, wn = w % WN;
-  const bf16* abase = a.a + (int64_t)b * a.a_rs + (int64_t)m0 * a.a_ld + (int64_t)s_begin * 64;
   // slab sl holds columns n0 + 64 sl of W (down), or of W_up (sl < NS / 2) and W_gate
   auto slab_col = [&](int sl) { return n0 + 64 * (GATED ? sl % (NS / 2) : sl); };
   auto slab_src = [&](int sl) {
-    return static_cast<const WT*>(a.w[GATED && sl >= NS / 2 ? 1 : 0]) + (int64_t)b * a.w_rs +
+    return static_cast<const WT*>(a.w[seg0][GATED && sl >= NS / 2 ? 1 : 0]) + (int64_t)b * a.w_rs[seg0] +
            (int64_t)s_begin * 64 * a.N;
   };
 
@@ -139,9 +148,10 @@ __global__ void __launch_bounds__(WM* WN * 64) k_readout_mm(const MmArgs a) {
     const int sl = is_row ? 0 : t - RT, c = slab_col(sl);
     // rows past the batch row's end read as zeros; columns past N read the next row (in range) or
     // zeros and are not stored
-    const char* p = is_row ? reinterpret_cast<const char*>(abase + (int64_t)t * 64 * a.a_ld)
-                           : reinterpret_cast<const char*>(slab_src(sl) + c);
-    const uint32_t n = is_row ? (uint32_t)max(0, min(64, a.rows - m0 - 64 * t)) * (uint32_t)a.a_ld * 2u
+    const int row = m0 + 64 * t, seg = seg_of(row), lr = row - seg_row(seg);
+    const bf16* rows = a.a[seg] + (int64_t)b * a.a_rs[seg] + (int64_t)lr * a.a_ld + (int64_t)s_begin * 64;
+    const char* p = is_row ? reinterpret_cast<const char*>(rows) : reinterpret_cast<const char*>(slab_src(sl) + c);
+    const uint32_t n = is_row ? (uint32_t)max(0, min(64, a.rows - lr)) * (uint32_t)a.a_ld * 2u
                               : (uint32_t)(64 * a.N - c) * 2u;
     const uint64_t u = reinterpret_cast<uint64_t>(p);
     src[i] = reinterpret_cast<const char*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)u) |
@@ -292,31 +302,34 @@ __global__ void __launch_bounds__(WM* WN * 64) k_readout_mm(const MmArgs a) {
   }
 
   // acc[i][j][e]: row m0 + rb + 32 i + acc_row(e)
-  if constexpr (GATED) {
-    const int col = n0 + 32 * wn + acc_col();
-    if (n0 + 32 * wn >= a.N) return;
-    bf16* h = a.h + (int64_t)b * a.rows_pad * a.N + col;
+  const int n1 = n0 + (GATED ? 32 : 64) * wn;  // this wave's first column
+  if (n1 >= a.N) return;
+  const int col = n1 + acc_col();
 #pragma unroll
-    for (int i = 0; i < MB; ++i) {
+  for (int i = 0; i < MB; ++i) {
+    const int row0 = m0 + rb + 32 * i;  // 32 rows of one segment
+    if (row0 >= m_end) continue;
+    const int seg = seg_of(row0), lr = row0 - seg_row(seg);
+    if constexpr (GATED) {
+      const int64_t base = ((int64_t)b * a.rows_pad + lr) * a.N + col;
+      bf16* h = a.h[seg] + base;
+      const bool keep = seg == 0 && a.u != nullptr;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int row = m0 + rb + 32 * i + acc_row(e);
         const float u = acc[i][0][e], g = acc[i][1][e];
-        if (row < a.rows_pad) h[(int64_t)row * a.N] = from_f32<bf16>((g * sigmoidf_acc(g)) * u);
+        const int64_t off = (int64_t)acc_row(e) * a.N;
+        h[off] = from_f32<bf16>((g * sigmoidf_acc(g)) * u);
+        if (keep) {
+          a.u[base + off] = u;
+          a.g[base + off] = g;
+        }
       }
-    }
-  } else {
-    float* z = a.zp + ((int64_t)split * a.B + b) * a.rows_pad * a.N + n0 + 64 * wn + acc_col();
-    if (n0 + 64 * wn >= a.N) return;
-#pragma unroll
-    for (int i = 0; i < MB; ++i) {
+    } else {
+      float* z = a.zp + ((((int64_t)seg * a.splits + split) * a.B + b) * a.rows_pad + lr) * a.N + col;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int row = m0 + rb + 32 * i + acc_row(e);
-        if (row < a.rows_pad) {
-          z[(int64_t)row * a.N] = acc[i][0][e];
-          z[(int64_t)row * a.N + 32] = acc[i][1][e];
-        }
+        z[(int64_t)acc_row(e) * a.N] = acc[i][0][e];
+        z[(int64_t)acc_row(e) * a.N + 32] = acc[i][1][e];
       }
     }
   }
@@ -378,10 +391,11 @@ MmPlan plan_mm(int64_t B, int64_t rows, int64_t cols, int64_t steps, int max_spl
 template <bool GATED, typename WT>
 void launch_mm(MmArgs m, MmPlan p, hipStream_t st) {
   const int cols = GATED ? 2 * m.N : m.N;
+  const int64_t matrices = m.joint ? m.B : (int64_t)m.B * m.nseg, rows = m.joint ? m.nseg * m.rows_pad : m.rows_pad;
   m.splits = p.splits;
-  m.mtiles = (int)ceil_div(m.rows_pad, tile_rows(p.tile));
+  m.mtiles = (int)ceil_div(rows, tile_rows(p.tile));
   m.ntiles = (int)ceil_div(cols, tile_cols(p.tile));
-  const dim3 grid((unsigned)((int64_t)m.B * m.splits * m.mtiles * m.ntiles));
+  const dim3 grid((unsigned)(matrices * m.splits * m.mtiles * m.ntiles));
   if (p.tile == kWide)
     hipLaunchKernelGGL((k_readout_mm<GATED, WT, 2, 4, 4, 2>), grid, dim3(512), 0, st, m);
   else if (p.tile == kMid)
@@ -398,15 +412,15 @@ MmPlan plan_down(int64_t B, int64_t T, int64_t D, int64_t F, bool w_fp32) {
 template <typename WT>
 void launch_both(const ReadoutMmArgs& a, hipStream_t st) {
   MmArgs m{};
-  m.B = a.B; m.rows = a.T; m.rows_pad = a.tok_pad; m.K = a.D; m.N = a.F;
-  m.a = static_cast<const bf16*>(a.x); m.a_rs = a.x_rs; m.a_ld = a.D;
-  m.w[0] = a.w_up; m.w[1] = a.w_gate; m.w_rs = a.w_rs;
-  m.h = static_cast<bf16*>(a.h);
+  m.B = a.B; m.nseg = 1; m.rows = a.T; m.rows_pad = a.tok_pad; m.K = a.D; m.N = a.F;
+  m.a[0] = static_cast<const bf16*>(a.x); m.a_rs[0] = a.x_rs; m.a_ld = a.D;
+  m.w[0][0] = a.w_up; m.w[0][1] = a.w_gate; m.w_rs[0] = a.w_rs;
+  m.h[0] = static_cast<bf16*>(a.h);
   launch_mm<true, WT>(m, plan_mm(a.B, a.tok_pad, 2 * (int64_t)a.F, a.D / 64, 1, a.w_fp32), st);
   MmArgs z{};
-  z.B = a.B; z.rows = a.tok_pad; z.rows_pad = a.tok_pad; z.K = a.F; z.N = a.D;
-  z.a = static_cast<const bf16*>(a.h); z.a_rs = (int64_t)a.tok_pad * a.F; z.a_ld = a.F;
-  z.w[0] = a.w_down; z.w[1] = nullptr; z.w_rs = a.w_rs;
+  z.B = a.B; z.nseg = 1; z.rows = a.tok_pad; z.rows_pad = a.tok_pad; z.K = a.F; z.N = a.D;
+  z.a[0] = static_cast<const bf16*>(a.h); z.a_rs[0] = (int64_t)a.tok_pad * a.F; z.a_ld = a.F;
+  z.w[0][0] = a.w_down; z.w_rs[0] = a.w_rs;
   z.zp = a.zp;
   launch_mm<false, WT>(z, plan_down(a.B, a.T, a.D, a.F, a.w_fp32), st);
 }
@@ -415,6 +429,42 @@ void launch_both(const ReadoutMmArgs& a, hipStream_t st) {
 
 int readout_mm_splits(int64_t B, int64_t T, int64_t D, int64_t F, bool w_fp32) {
   return plan_down(B, T, D, F, w_fp32).splits;
+}
+
+static MmPlan plan_update_down(int64_t B, int64_t T, int64_t D, int64_t F, bool joint, int most) {
+  const int64_t rows = ceil_div(T, 64) * 64;
+  return plan_mm(joint ? B : 2 * B, joint ? 2 * rows : rows, D, F / 64,
+                 (int)std::min<int64_t>(std::min(most, kMaxSplits), F / 64), true);
+}
+
+int update_mm_splits(int64_t B, int64_t T, int64_t D, int64_t F, bool joint, int most) {
+  return plan_update_down(B, T, D, F, joint, most).splits;
+}
+
+void launch_update_up(const UpdateMmArgs& a, bool joint, hipStream_t st) {
+  MmArgs m{};
+  m.B = a.B; m.nseg = 2; m.joint = joint; m.rows = a.T; m.rows_pad = a.tok_pad; m.K = a.D; m.N = a.F;
+  m.a_ld = a.D;
+  for (int s = 0; s < 2; ++s) {
+    m.a[s] = static_cast<const bf16*>(a.x[s]); m.a_rs[s] = a.x_rs[s];
+    m.w[s][0] = a.w_up[s]; m.w[s][1] = a.w_gate[s]; m.w_rs[s] = a.w_rs[s];
+    m.h[s] = static_cast<bf16*>(a.h[s]);
+  }
+  m.u = a.u_store; m.g = a.g_store;
+  launch_mm<true, float>(m, plan_mm(joint ? a.B : 2 * a.B, joint ? 2 * a.tok_pad : a.tok_pad, 2 * (int64_t)a.F,
+                                    a.D / 64, 1, true), st);
+}
+
+void launch_update_down(const UpdateMmArgs& a, bool joint, hipStream_t st) {
+  MmArgs z{};
+  z.B = a.B; z.nseg = 2; z.joint = joint; z.rows = a.tok_pad; z.rows_pad = a.tok_pad; z.K = a.F; z.N = a.D;
+  z.a_ld = a.F;
+  for (int s = 0; s < 2; ++s) {
+    z.a[s] = static_cast<const bf16*>(a.h[s]); z.a_rs[s] = (int64_t)a.tok_pad * a.F;
+    z.w[s][0] = a.w_down[s]; z.w_rs[s] = a.w_rs[s];
+  }
+  z.zp = a.zp;
+  launch_mm<false, float>(z, plan_update_down(a.B, a.T, a.D, a.F, joint, a.splits), st);
 }
 
 void launch_readout_mm(const ReadoutMmArgs& a, hipStream_t st) {

@@ -30,9 +30,7 @@ struct LnGradArgs {
 // kPer features per thread (D <= 256 kPer); the split partials of a token are read
 // 16 / kPer splits at a time so that many loads are in flight together.
 template <typename T, int kPer>
-__global__ void __launch_bounds__(kThreads) k_ln_grad(const LnGradArgs a) {
-  __shared__ float red[4];
-  const int t = blockIdx.x, b = blockIdx.y;
+__device__ __forceinline__ void ln_grad_row(const LnGradArgs& a, int t, int b, float* red, float* red2) {
   T* dz = static_cast<T*>(a.dz) + ((int64_t)b * a.tok_pad + t) * a.D;
   if (t >= a.C) {
     for (int d = threadIdx.x; d < a.D; d += kThreads) dz[d] = from_f32<T>(0.f);
@@ -96,7 +94,6 @@ __global__ void __launch_bounds__(kThreads) k_ln_grad(const LnGradArgs a) {
     }
   }
   // the loss and the mask's token count in one reduction
-  __shared__ float red2[8];
   const float* mr = a.mask != nullptr ? a.mask + (int64_t)b * a.mask_rs : nullptr;
   float msum = 0.f;  // the chunk's valid tokens (C may exceed the workgroup)
   if (mr != nullptr)
@@ -134,6 +131,12 @@ __global__ void __launch_bounds__(kThreads) k_ln_grad(const LnGradArgs a) {
     if (d < a.D) dz[d] = from_f32<T>(rstd * (e[i] - m1 - z[i] * m2));
   }
   if (threadIdx.x == 0) a.loss[b * a.tok_pad + t] = a.mask != nullptr ? token_loss * m_t : token_loss;
+}
+
+template <typename T, int kPer>
+__global__ void __launch_bounds__(kThreads) k_ln_grad(const LnGradArgs a) {
+  __shared__ float red[4], red2[8];
+  ln_grad_row<T, kPer>(a, blockIdx.x, blockIdx.y, red, red2);
 }
 
 // Launch k_ln_grad with the narrowest per-thread width that covers d_model.

@@ -1,0 +1,375 @@
+// Backward pass and state write of one bf16 chunk update (reference fused_chunk_ttt_step,
+// model/uttt_layer.py:279-534), gfx950 (MI355X): operands straight into LDS, fp32 state.
+//
+//   k_update_back   dH = dZ W_down^T per F tile, dU, dG, and the tile's squared gradient norm
+//   k_update_write  one 64 x 64 gradient tile from the chunk's token slabs, then S' = beta S - c g,
+//                   W' = decay W + S' (or only the tile's squared norm)
+//
+// The write is bound by the state it streams (48 D F bytes per row), the backward pass by the
+// latency of its D loop on few workgroups.  Measured against the register-staged kernels they
+// replaced (backward with the norm / state write with the row scalars, us):
+//   1 row x 37 tokens, d 768, F 2048      26 -> 14 / 23 -> 18
+//   8 rows x 64 tokens, d 768, F 2048     32 -> 17 / 163 -> 123 (604 MB, 4.9 TB/s)
+//   4 rows x 64 tokens, d 2048, F 5504    89 -> 40 / 569 -> 415 (5.2 TB/s)
+//   2 rows x 128 tokens, d 1024, F 2816   55 -> 26 / 146 -> 61
+#include "update_mm.h"
+
+#include "uttt_device.h"
+
+namespace uttt {
+namespace {
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // the caller's outputs: any fp32 alignment
+
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
+}
+__device__ __forceinline__ void lds_write_b64(uint32_t addr, uint2 v) {
+  asm volatile("ds_write_b64 %0, %1" ::"v"(addr), "v"(v));
+}
+
+// the four k pieces of rows rb .. rb + 31 of a row tile
+__device__ __forceinline__ void row_frags(uint32_t tile, int rb, int lane, bf16x8 (&f)[4]) {
+#pragma unroll
+  for (int s = 0; s < 4; ++s) f[s] = lds_read_bf16x8<0>(row_frag_addr(tile, rb, lane, s));
+}
+template <int AHEAD>
+__device__ __forceinline__ void wait_frags(bf16x8 (&f)[4]) {
+  asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]) : "n"(AHEAD));
+}
+__device__ __forceinline__ void mma4(f32x16& acc, const bf16x8 (&a)[4], const bf16x8 (&b)[4]) {
+#pragma unroll
+  for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s], b[s], acc, 0, 0, 0);
+}
+
+// One (F tile, row, token block).  NORM (one token block): the tile's squared gradient norm from
+// Gram matrices, |K^T dU|^2 = <K K^T, dU dU^T> (and alike for dG; |H^T dZ|^2 = <H H^T, dZ dZ^T>):
+// K K^T and dZ dZ^T accumulate over D beside dH from the tiles dH needs anyway, where forming the
+// gradient tiles took a second loop over D with three products and transposes per step.  Sums of
+// 64 x 64 products of fp32 accumulations; the clip factor's relative error stays near 1e-6.
+template <bool NORM>
+__global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArgs a) {
+  constexpr int TILES = NORM ? 2 : 1;        // dZ rows (and K rows) by direct loads
+  constexpr int SLOT = (TILES + 1) * 8192;   // then the W_down rows, rounded through registers
+  constexpr int PER = TILES * 2, WCH = 4;    // loads per wave and step, W_down pieces per thread
+  constexpr int SLOTS = 3;
+  __shared__ __align__(1024) char ring[SLOTS * SLOT];
+  __shared__ __align__(1024) char htile[NORM ? 8192 : 16];
+  const int nF = a.F / 64;
+  const RowTile rt = row_tile(blockIdx.x, a.B, nF * a.ntb);
+  if (!rt.valid) return;
+  const int b = rt.b, ft = rt.tile % nF, t0 = (rt.tile / nF) * 64, f0 = ft * 64;
+  const int w = uniform((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wr = (w >> 1) * 32, wc = (w & 1) * 32;
+  const bf16* dz = static_cast<const bf16*>(a.dz) + ((int64_t)b * a.tok_pad + t0) * a.D;
+  const bf16* kr = static_cast<const bf16*>(a.k) + (int64_t)b * a.k_rs + (int64_t)t0 * a.D;
+  const float* wd = a.w_down + (int64_t)b * a.D * a.F + (int64_t)f0 * a.D;
+  const int64_t rowbase = ((int64_t)b * a.tok_pad + t0) * a.F + f0;
+  const uint32_t ring0 = lds_addr(ring), h0 = lds_addr(htile);
+  const uint32_t k_bytes = (uint32_t)uniform(max(0, min(64, a.C - t0)) * a.D * 2);
+
+  int voff[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) voff[i] = row_src_off(w + 4 * i, lane, a.D);
+  auto issue = [&](int step, int at) {
+    const uint32_t base = ring0 + (uint32_t)((at % SLOTS) * SLOT);
+    const __amdgpu_buffer_rsrc_t rz = buffer_rsrc(dz + step * 64, (uint32_t)(64 * a.D * 2));
+    const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(kr + step * 64, k_bytes);  // rows past C read as zeros
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      buffer_load_lds_raw(rz, lds_ptr(base + (uint32_t)((w + 4 * i) * 1024)), 16, voff[i], 0, 0, 0);
+      if constexpr (NORM)
+        buffer_load_lds_raw(rk, lds_ptr(base + 8192u + (uint32_t)((w + 4 * i) * 1024)), 16, voff[i], 0, 0, 0);
+    }
+  };
+  // W_down rows: thread's piece i is row 16 i + tid / 16, columns 4 (tid % 16) .. + 3
+  struct Pieces {
+    f32x4 r[WCH];
+  };
+  const int wrow = (int)threadIdx.x >> 4, wc4 = threadIdx.x & 15;
+  const int wsrc = (wrow * a.D + 4 * wc4) * 4;
+  const uint32_t wdst =
+      ring0 + (uint32_t)(TILES * 8192 + wrow * 128 + (((wc4 >> 1) ^ row_swz(wrow)) * 16) + (wc4 & 1) * 8);
+  auto wload = [&](Pieces& p, int step) {
+    const __amdgpu_buffer_rsrc_t r = buffer_rsrc(wd + step * 64, (uint32_t)(64 * a.D - step * 64) * 4u);
+#pragma unroll
+    for (int i = 0; i < WCH; ++i)
+      p.r[i] =
+          __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, wsrc, 16 * i * a.D * 4, 0));
+  };
+  auto wstore = [&](const Pieces& p, int step) {
+    const uint32_t base = wdst + (uint32_t)((step % SLOTS) * SLOT);
+#pragma unroll
+    for (int i = 0; i < WCH; ++i)  // 16 rows on, the row's swizzle is the same
+      lds_write_b64(base + (uint32_t)(i * 2048),
+                    make_uint2(pack_bf16(p.r[i][0], p.r[i][1]), pack_bf16(p.r[i][2], p.r[i][3])));
+  };
+
+  if constexpr (NORM) {
+    const __amdgpu_buffer_rsrc_t rh =
+        buffer_rsrc(static_cast<const bf16*>(a.h) + rowbase, (uint32_t)(64 * a.F * 2));
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      buffer_load_lds_raw(rh, lds_ptr(h0 + (uint32_t)((w + 4 * i) * 1024)), 16, row_src_off(w + 4 * i, lane, a.F), 0,
+                          0, 0);
+  }
+  const int nsteps = a.D / 64, last = nsteps - 1;
+  Pieces p0, p1;
+  wload(p0, 0);
+  issue(0, 0);
+  wload(p1, min(1, last));
+  issue(min(1, last), 1);
+  wstore(p0, 0);
+  f32x16 dh, zz, kk;
+  zero(dh);
+  zero(zz);
+  zero(kk);
+  // loads run two steps ahead (the last steps load the last step again, so that every iteration has
+  // the same loads in flight); a step's W_down pieces reach LDS during the step before it
+  auto body = [&](int step, Pieces& mine, Pieces& next) {
+    wait_vmcnt<WCH + PER>();
+    asm volatile("s_waitcnt lgkmcnt(0)");
+    __builtin_amdgcn_s_barrier();
+    wload(mine, min(step + 2, last));
+    issue(min(step + 2, last), step + 2);
+    const uint32_t so = ring0 + (uint32_t)((step % SLOTS) * SLOT);
+    bf16x8 fa[4], fb[4];
+    row_frags(so, wr, lane, fa);
+    row_frags(so + TILES * 8192u, wc, lane, fb);
+    wait_frags<4>(fa);
+    wait_frags<0>(fb);
+    mma4(dh, fa, fb);
+    if constexpr (NORM) {
+      row_frags(so, wc, lane, fb);
+      wait_frags<0>(fb);
+      mma4(zz, fa, fb);
+      row_frags(so + 8192u, wr, lane, fa);
+      row_frags(so + 8192u, wc, lane, fb);
+      wait_frags<4>(fa);
+      wait_frags<0>(fb);
+      mma4(kk, fa, fb);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    wstore(next, step + 1);
+  };
+  int step = 0;
+  for (; step + 2 <= nsteps; step += 2) {
+    body(step, p0, p1);
+    body(step + 1, p1, p0);
+  }
+  if (step < nsteps) body(step, p0, p1);
+  wait_vmcnt<0>();
+  asm volatile("s_waitcnt lgkmcnt(0)");
+  float uv[16], gv[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int64_t off = rowbase + (int64_t)(wr + acc_row(i)) * a.F + wc + acc_col();
+    uv[i] = a.u[off];
+    gv[i] = a.g[off];
+  }
+  __syncthreads();  // the ring is free: dU and dG row tiles go to its first two tiles
+
+  bf16* dus = reinterpret_cast<bf16*>(ring);
+  bf16* dgs = reinterpret_cast<bf16*>(ring + 8192);
+  const int f = wc + acc_col();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int t = wr + acc_row(i);
+    const float u = uv[i], g = gv[i], sg = sigmoidf_acc(g);
+    const bf16 du = from_f32<bf16>(dh[i] * (g * sg));
+    const bf16 dg = from_f32<bf16>(dh[i] * u * (sg * (1.0f + g * (1.0f - sg))));
+    const int64_t off = rowbase + (int64_t)t * a.F + f;
+    static_cast<bf16*>(a.du)[off] = du;
+    static_cast<bf16*>(a.dg)[off] = dg;
+    if constexpr (NORM) {
+      const int at = t * 64 + (((f >> 3) ^ row_swz(t)) * 8) + (f & 7);
+      dus[at] = du;
+      dgs[at] = dg;
+    }
+  }
+  if constexpr (NORM) {
+    __syncthreads();
+    f32x16 g1, g2;
+    zero(g1);
+    zero(g2);
+    bf16x8 fa[4], fb[4];
+    row_frags(ring0, wr, lane, fa);
+    row_frags(ring0, wc, lane, fb);
+    wait_frags<4>(fa);
+    wait_frags<0>(fb);
+    mma4(g1, fa, fb);
+    row_frags(ring0 + 8192u, wr, lane, fa);
+    row_frags(ring0 + 8192u, wc, lane, fb);
+    wait_frags<4>(fa);
+    wait_frags<0>(fb);
+    mma4(g1, fa, fb);
+    row_frags(h0, wr, lane, fa);
+    row_frags(h0, wc, lane, fb);
+    wait_frags<4>(fa);
+    wait_frags<0>(fb);
+    mma4(g2, fa, fb);
+    float sq = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sq += kk[i] * g1[i] + zz[i] * g2[i];
+    // the scratch of the sum: the ring past the two tiles (160 KB of LDS hold two workgroups)
+    const float total = block_sum(sq, reinterpret_cast<float*>(ring + 16384));
+    if (threadIdx.x == 0) a.nrm[b * nF + ft] = total;
+  }
+}
+
+// One 64 x 64 tile of one matrix: the gradient from the chunk's token slabs (tokens down the rows:
+// transposing reads for both operands), then the state, whose 16-byte pieces were in flight
+// meanwhile; the gradient tile crosses LDS so that they stay whole rows of 256 bytes.
+template <bool NORM>
+__global__ void __launch_bounds__(kThreads) k_update_write(const UpdateWriteArgs a) {
+  constexpr int GLD = 68;  // floats per gradient tile row in LDS
+  __shared__ __align__(1024) char ring[2 * 16384];  // two steps of one token block: A slab, B slab
+  __shared__ float red[4];
+  static_assert(64 * GLD * 4 <= sizeof(ring), "the gradient tile reuses the ring");
+  const int nD = a.D / 64, nF = a.F / 64, per = nD * nF;
+  const RowTile rt = row_tile(blockIdx.x, a.B, 3 * per);
+  if (!rt.valid) return;
+  const int b = rt.b, m = rt.tile / per, j = rt.tile - m * per;
+  const int w = uniform((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int wr = (w >> 1) * 32, wc = (w & 1) * 32;
+  int r0, c0, ld_out, a_ld, b_ld, a_rows;
+  const bf16 *as, *bs;
+  if (m < 2) {  // W_up / W_gate tile (d, f) = K^T dU / K^T dG
+    r0 = (j / nF) * 64;
+    c0 = (j - (j / nF) * nF) * 64;
+    ld_out = a.F;
+    as = static_cast<const bf16*>(a.k) + (int64_t)b * a.k_rs + r0;
+    a_ld = a.D;
+    a_rows = a.C;
+    bs = static_cast<const bf16*>(m == 0 ? a.du : a.dg) + (int64_t)b * a.tok_pad * a.F + c0;
+    b_ld = a.F;
+  } else {  // W_down tile (f, d) = H^T dZ
+    r0 = (j / nD) * 64;
+    c0 = (j - (j / nD) * nD) * 64;
+    ld_out = a.D;
+    as = static_cast<const bf16*>(a.h) + (int64_t)b * a.tok_pad * a.F + r0;
+    a_ld = a.F;
+    a_rows = a.tok_pad;  // rows past the chunk are zero
+    bs = static_cast<const bf16*>(a.dz) + (int64_t)b * a.tok_pad * a.D + c0;
+    b_ld = a.D;
+  }
+  const uint32_t ring0 = lds_addr(ring);
+  int aoff[2], boff[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    aoff[i] = slab_src_off(w + 4 * i, lane, a_ld);
+    boff[i] = slab_src_off(w + 4 * i, lane, b_ld);
+  }
+  auto issue = [&](int tb) {
+    const uint32_t base = ring0 + (uint32_t)((tb & 1) * 16384);
+    const int rows = max(0, min(64, a_rows - 64 * tb));
+    // the slabs' columns end 2 r0 (2 c0) bytes before their rows' next columns: ranges to the last row's end
+    const __amdgpu_buffer_rsrc_t ra =
+        buffer_rsrc(as + (int64_t)tb * 64 * a_ld, (uint32_t)uniform(rows > 0 ? (rows * a_ld - r0) * 2 : 0));
+    const __amdgpu_buffer_rsrc_t rb = buffer_rsrc(bs + (int64_t)tb * 64 * b_ld, (uint32_t)((64 * b_ld - c0) * 2));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      buffer_load_lds_raw(ra, lds_ptr(base + (uint32_t)((w + 4 * i) * 1024)), 16, aoff[i], 0, 0, 0);
+      buffer_load_lds_raw(rb, lds_ptr(base + 8192u + (uint32_t)((w + 4 * i) * 1024)), 16, boff[i], 0, 0, 0);
+    }
+  };
+  issue(0);
+  if (a.ntb > 1) issue(1);
+  // the state tile is the bulk of the traffic: its loads go out before the products
+  const int64_t mat = (int64_t)a.D * a.F;
+  const int row = (int)threadIdx.x >> 4, c4 = threadIdx.x & 15;
+  const int64_t at = (int64_t)b * mat + (int64_t)(r0 + row) * ld_out + c0 + 4 * c4;
+  f32x4 wv[4], sv[4];
+  float clip = 0.f, decay = 0.f, act = 0.f;
+  if constexpr (!NORM) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      wv[i] = *reinterpret_cast<const f32x4*>(a.w[m] + at + (int64_t)16 * i * ld_out);
+      sv[i] = *reinterpret_cast<const f32x4*>(a.s[m] + at + (int64_t)16 * i * ld_out);
+    }
+    clip = a.scalars[4 * b];
+    decay = a.scalars[4 * b + 1];
+    act = a.scalars[4 * b + 2];
+  }
+  f32x16 acc;
+  zero(acc);
+  const uint32_t ta = slab_tr_addr(ring0, wr, lane), tb0 = slab_tr_addr(ring0 + 8192u, wc, lane);
+  for (int tb = 0; tb < a.ntb; ++tb) {
+    if (tb == 0) {
+      // block 0's loads are the oldest; block 1's and the state's may still be in flight
+      if (a.ntb > 1)
+        wait_vmcnt<NORM ? 4 : 12>();
+      else
+        wait_vmcnt<NORM ? 0 : 8>();
+    } else {
+      wait_vmcnt<0>();
+    }
+    __builtin_amdgcn_s_barrier();
+    const uint32_t so = (uint32_t)((tb & 1) * 16384);
+    bf16x8 fa[4], fb[4];
+    slab_frags(ta + so, fa);
+    slab_frags(tb0 + so, fb);
+    lds_wait_frags(fa, fb);
+    mma4(acc, fa, fb);
+    if (tb + 2 < a.ntb) {
+      __builtin_amdgcn_s_barrier();  // every wave is done with this slot
+      issue(tb + 2);
+    }
+  }
+  if constexpr (NORM) {
+    float sq = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sq += acc[i] * acc[i];
+    const float total = block_sum(sq, red);
+    if (threadIdx.x == 0) a.nrm[(int64_t)b * 3 * per + rt.tile] = total;
+    return;
+  }
+  __builtin_amdgcn_s_barrier();  // the slabs are consumed: the gradient tile takes their place
+  float* gt = reinterpret_cast<float*>(ring);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) gt[(wr + acc_row(i)) * GLD + wc + acc_col()] = acc[i];
+  __syncthreads();
+  const bool active = act != 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4 g = *reinterpret_cast<const f32x4*>(gt + (row + 16 * i) * GLD + 4 * c4);
+    f32x4 wn, sn;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+#pragma clang fp contract(off)
+      const float step = g[e] * clip;
+      const float s_new = a.beta * sv[i][e] - step;
+      const float w_new = decay * wv[i][e] + s_new;
+      wn[e] = active ? w_new : wv[i][e];
+      sn[e] = active ? s_new : sv[i][e];
+    }
+    *reinterpret_cast<f32x4u*>(a.w_out[m] + at + (int64_t)16 * i * ld_out) = wn;
+    *reinterpret_cast<f32x4u*>(a.s_out[m] + at + (int64_t)16 * i * ld_out) = sn;
+  }
+}
+
+}  // namespace
+
+void launch_update_back(const UpdateBackArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)row_tile_blocks(a.B, (a.F / 64) * a.ntb));
+  if (a.ntb == 1)
+    hipLaunchKernelGGL(k_update_back<true>, grid, dim3(kThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL(k_update_back<false>, grid, dim3(kThreads), 0, st, a);
+}
+
+void launch_update_norm(const UpdateWriteArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(k_update_write<true>, dim3((unsigned)row_tile_blocks(a.B, 3 * (a.D / 64) * (a.F / 64))),
+                     dim3(kThreads), 0, st, a);
+}
+
+void launch_update_write(const UpdateWriteArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(k_update_write<false>, dim3((unsigned)row_tile_blocks(a.B, 3 * (a.D / 64) * (a.F / 64))),
+                     dim3(kThreads), 0, st, a);
+}
+
+}  // namespace uttt
