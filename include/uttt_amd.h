@@ -344,6 +344,21 @@ typedef struct {
 
 int uttt_rope_kv_append(const uttt_rope_append_args* args, uttt_stream_t stream);
 
+/* The same with a bounded cache around the call (model/uttt_layer.py:1082-1114), in one launch: the
+ * last `history` rows of an earlier cache go to [kv_offset - history, kv_offset) of k_cache / v_cache,
+ * and rows [kv_offset + tokens - out_len, kv_offset + tokens) of them (history rows first) also go to
+ * k_out / v_out.  Both optional (history 0, out_len 0).  Needs 16-byte aligned pointers and strides in
+ * whole 16-byte pieces, head_dim a multiple of 16 (bf16) or 8 (fp32), and no folded norm. */
+typedef struct {
+  const void* k_hist; int64_t k_hist_stride_b, k_hist_stride_h, k_hist_stride_t; /* first of the last `history` rows */
+  const void* v_hist; int64_t v_hist_stride_b, v_hist_stride_h, v_hist_stride_t;
+  int64_t history;
+  void* k_out; void* v_out; int64_t out_stride_b, out_stride_h, out_stride_t;
+  int64_t out_len;
+} uttt_kv_roll_args;
+
+int uttt_rope_kv_roll(const uttt_rope_append_args* args, const uttt_kv_roll_args* roll, uttt_stream_t stream);
+
 /* ---------------------------------------------------------------------------
  * 4. Sliding-window GQA attention for prefill / multi-token steps.
  *    Replaces the SDPA / FlexAttention dispatch of SlidingWindowAttention.forward

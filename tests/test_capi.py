@@ -40,7 +40,7 @@ def test_every_declared_symbol_is_exported_and_typed(lib):
 
 def test_struct_layouts_match_the_c_header(tmp_path):
     structs = {"uttt_chunk_update_args": N.ChunkUpdateArgs, "uttt_readout_args": N.ReadoutArgs,
-               "uttt_rope_append_args": N.RopeAppendArgs, "uttt_swa_prefill_args": N.SwaPrefillArgs,
+               "uttt_rope_append_args": N.RopeAppendArgs, "uttt_kv_roll_args": N.KvRollArgs, "uttt_swa_prefill_args": N.SwaPrefillArgs,
                "uttt_swa_decode_args": N.SwaDecodeArgs, "uttt_elastic_pull_args": N.ElasticPullArgs,
                "uttt_chunk_chain_args": N.ChunkChainArgs, "uttt_proj_epilogue_args": N.ProjEpilogueArgs,
                "uttt_skinny_linear_args": N.SkinnyLinearArgs, "uttt_greedy_args": N.GreedyArgs,

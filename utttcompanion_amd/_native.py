@@ -167,6 +167,16 @@ class RopeAppendArgs(C.Structure):
     ]
 
 
+class KvRollArgs(C.Structure):
+    _fields_ = [
+        ("k_hist", _P), ("k_hist_stride_b", _I64), ("k_hist_stride_h", _I64), ("k_hist_stride_t", _I64),
+        ("v_hist", _P), ("v_hist_stride_b", _I64), ("v_hist_stride_h", _I64), ("v_hist_stride_t", _I64),
+        ("history", _I64),
+        ("k_out", _P), ("v_out", _P), ("out_stride_b", _I64), ("out_stride_h", _I64), ("out_stride_t", _I64),
+        ("out_len", _I64),
+    ]
+
+
 class SwaPrefillArgs(C.Structure):
     _fields_ = [
         ("batch", _I64), ("n_heads", _I64), ("n_kv_heads", _I64), ("q_len", _I64), ("kv_len", _I64),
@@ -253,6 +263,7 @@ SIGNATURES = {
     "uttt_readout_workspace": (C.c_size_t, [_I64, _I64, _I64, _I64, _I32]),
     "uttt_swiglu_readout": (C.c_int, [C.POINTER(ReadoutArgs), _P, C.c_size_t, _P]),
     "uttt_rope_kv_append": (C.c_int, [C.POINTER(RopeAppendArgs), _P]),
+    "uttt_rope_kv_roll": (C.c_int, [C.POINTER(RopeAppendArgs), C.POINTER(KvRollArgs), _P]),
     "uttt_swa_prefill_workspace": (C.c_size_t, [_I64, _I64, _I64, _I64, _I64, _I64]),
     "uttt_swa_prefill": (C.c_int, [C.POINTER(SwaPrefillArgs), _P]),
     "uttt_swa_decode_workspace": (C.c_size_t, [_I64, _I64, _I64, _I64, _I64]),

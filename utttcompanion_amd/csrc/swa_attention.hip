@@ -116,6 +116,102 @@ __global__ void __launch_bounds__(kThreads) k_rope_append(const uttt_rope_append
   }
 }
 
+// The same in 16-byte pieces (pointers and strides allowing), with the cache around the call: history
+// rows copied in front of the appended ones, and the last out_len rows copied to a new cache.
+// Without a folded norm the pieces of all tokens and history rows of a row form one list, a piece
+// per thread (XN: a workgroup per token, whose threads first meet for the row's scale).  Bound by the
+// bytes: 4 x 4096 tokens, 16 + 2 x 4 heads of 128: 65 us a token row per workgroup in 2-byte
+// accesses, 45 us so, and the cache copies (11 us in two launches, 17 in four with history) gone.
+template <typename T> struct Piece16;
+template <> struct Piece16<bf16> { using type = bf16x8; };
+template <> struct Piece16<float> { using type = f32x4; };
+
+template <typename T, bool XN>
+__global__ void __launch_bounds__(kThreads) k_rope_roll(const uttt_rope_append_args a, const uttt_kv_roll_args c) {
+  using V = typename Piece16<T>::type;
+  constexpr int VEC = 16 / (int)sizeof(T);
+  const int b = blockIdx.y, hd = (int)a.head_dim, half = hd / 2;
+  const int ph = half / VEC, pr = hd / VEC;  // rotated pairs of pieces per head, pieces per head
+  const int nq = (int)a.n_heads * ph, nk = (int)a.n_kv_heads * ph, nv = (int)a.n_kv_heads * pr;
+  const int per_tok = nq + nk + nv, per_hist = 2 * nv;
+  const int64_t first_out = a.kv_offset + a.tokens - c.out_len;  // KV index of the new cache's first row
+  float xs = 1.0f;
+  if constexpr (XN) {
+    __shared__ float red[4];
+    const T* xr = static_cast<const T*>(a.x) + b * a.x_stride_b + (int64_t)blockIdx.x * a.x_stride_t;
+    float ss = 0.f;
+    for (int i = threadIdx.x; i < a.x_dim; i += kThreads) {
+      const float xv = to_f32(xr[i]);
+      ss += xv * xv;
+    }
+    xs = 1.0f / sqrtf(block_sum(ss, red) / (float)a.x_dim + a.x_eps);
+  }
+  auto put = [&](bool is_k, int h, int64_t row, int e, const V& v) {  // a KV row's piece into both caches
+    const int64_t at = b * a.kv_stride_b + h * a.kv_stride_h + row * a.kv_stride_t + e;
+    *reinterpret_cast<V*>(static_cast<T*>(is_k ? a.k_cache : a.v_cache) + at) = v;
+    if (c.out_len > 0 && row >= first_out)
+      *reinterpret_cast<V*>(static_cast<T*>(is_k ? c.k_out : c.v_out) + b * c.out_stride_b + h * c.out_stride_h +
+                            (row - first_out) * c.out_stride_t + e) = v;
+  };
+  auto token_piece = [&](int t, int u) {
+    if (u < nq + nk) {
+      const bool is_q = u < nq;
+      const int i = is_q ? u : u - nq, h = i / ph, e = (i - h * ph) * VEC;
+      T* qh = static_cast<T*>(a.q) + b * a.q_stride_b + t * a.q_stride_t + h * a.q_stride_h;
+      const T* src = is_q ? qh : static_cast<const T*>(a.k) + b * a.k_stride_b + t * a.k_stride_t + h * a.k_stride_h;
+      const V lo = *reinterpret_cast<const V*>(src + e), hi = *reinterpret_cast<const V*>(src + e + half);
+      const float* cr = a.cos_table + (a.start_pos + t) * hd + e;
+      const float* sr = a.sin_table + (a.start_pos + t) * hd + e;
+      float cv[VEC], sv[VEC];
+#pragma unroll
+      for (int j = 0; j < VEC; j += 4) {
+        *reinterpret_cast<f32x4*>(cv + j) = *reinterpret_cast<const f32x4*>(cr + j);
+        *reinterpret_cast<f32x4*>(sv + j) = *reinterpret_cast<const f32x4*>(sr + j);
+      }
+      V ol, oh;
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        T x, y;
+        rope_pair<T>(xs * to_f32((T)lo[j]), xs * to_f32((T)hi[j]), cv[j], sv[j], x, y);
+        ol[j] = x;
+        oh[j] = y;
+      }
+      if (is_q) {
+        *reinterpret_cast<V*>(qh + e) = ol;
+        *reinterpret_cast<V*>(qh + e + half) = oh;
+      } else {
+        put(true, h, a.kv_offset + t, e, ol);
+        put(true, h, a.kv_offset + t, e + half, oh);
+      }
+    } else {
+      const int i = u - nq - nk, h = i / pr, e = (i - h * pr) * VEC;
+      V v = *reinterpret_cast<const V*>(static_cast<const T*>(a.v) + b * a.v_stride_b + t * a.v_stride_t +
+                                        h * a.v_stride_h + e);
+      if constexpr (XN) {
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) v[j] = from_f32<T>(xs * to_f32((T)v[j]));
+      }
+      put(false, h, a.kv_offset + t, e, v);
+    }
+  };
+  if constexpr (XN) {
+    for (int u = threadIdx.x; u < per_tok; u += kThreads) token_piece(blockIdx.x, u);
+  } else {
+    const int64_t idx = (int64_t)blockIdx.x * kThreads + threadIdx.x, n_tok = a.tokens * per_tok;
+    if (idx < n_tok) {
+      token_piece((int)(idx / per_tok), (int)(idx % per_tok));
+    } else if (idx - n_tok < c.history * per_hist) {
+      const int64_t i = idx - n_tok, j = i / per_hist;
+      const int u = (int)(i - j * per_hist);
+      const bool is_k = u < nv;
+      const int w = is_k ? u : u - nv, h = w / pr, e = (w - h * pr) * VEC;
+      const T* src = is_k ? static_cast<const T*>(c.k_hist) + b * c.k_hist_stride_b + h * c.k_hist_stride_h + j * c.k_hist_stride_t
+                          : static_cast<const T*>(c.v_hist) + b * c.v_hist_stride_b + h * c.v_hist_stride_h + j * c.v_hist_stride_t;
+      put(is_k, h, a.kv_offset - c.history + j, e, *reinterpret_cast<const V*>(src + e));
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Prefill.  grid (q tiles of 64, n_heads, batch * nsplit): the key tiles that intersect a
 // q tile's window are divided among `nsplit` workgroups; each wave owns 16 queries.  With
@@ -1019,7 +1115,7 @@ static void launch_decode(const uttt_swa_decode_args& a, hipStream_t st) {
 
 using namespace uttt;
 
-extern "C" int uttt_rope_kv_append(const uttt_rope_append_args* a, uttt_stream_t stream) {
+static int validate_rope(const uttt_rope_append_args* a) {
   UTTT_REQUIRE(a != nullptr, "args is NULL");
   UTTT_REQUIRE(a->batch >= 1 && a->batch <= 65535 && a->tokens >= 1, "batch/tokens out of range");
   UTTT_REQUIRE(a->head_dim >= 2 && a->head_dim % 2 == 0, "head_dim must be even");
@@ -1032,13 +1128,72 @@ extern "C" int uttt_rope_kv_append(const uttt_rope_append_args* a, uttt_stream_t
   UTTT_REQUIRE(a->kv_offset >= 0, "kv_offset must be >= 0");
   UTTT_REQUIRE(a->act_dtype == UTTT_DTYPE_F32 || a->act_dtype == UTTT_DTYPE_BF16, "bad act_dtype");
   UTTT_REQUIRE(a->x == nullptr || (a->x_dim >= 1 && a->x_eps > 0.f), "a folded norm needs x_dim >= 1 and x_eps > 0");
+  return UTTT_OK;
+}
+
+// Whether every access of the 16-byte form is one aligned piece, and its list fits one grid.
+static bool rope_in_pieces(const uttt_rope_append_args& a, const uttt_kv_roll_args& c) {
+  const int64_t v = a.act_dtype == UTTT_DTYPE_BF16 ? 8 : 4;
+  auto whole = [v](int64_t x, int64_t y, int64_t z) { return x % v == 0 && y % v == 0 && z % v == 0; };
+  const int64_t pieces = (a.n_heads + 4 * a.n_kv_heads) * (a.head_dim / v + 1) * (a.tokens + c.history);
+  return a.head_dim % (2 * v) == 0 && pieces < (1LL << 31) && aligned16(a.cos_table) && aligned16(a.sin_table) &&
+         aligned16(a.q) && aligned16(a.k) && aligned16(a.v) && aligned16(a.k_cache) && aligned16(a.v_cache) &&
+         whole(a.q_stride_b, a.q_stride_t, a.q_stride_h) && whole(a.k_stride_b, a.k_stride_t, a.k_stride_h) &&
+         whole(a.v_stride_b, a.v_stride_t, a.v_stride_h) && whole(a.kv_stride_b, a.kv_stride_h, a.kv_stride_t) &&
+         (c.history == 0 || (aligned16(c.k_hist) && aligned16(c.v_hist) &&
+                             whole(c.k_hist_stride_b, c.k_hist_stride_h, c.k_hist_stride_t) &&
+                             whole(c.v_hist_stride_b, c.v_hist_stride_h, c.v_hist_stride_t))) &&
+         (c.out_len == 0 || (aligned16(c.k_out) && aligned16(c.v_out) &&
+                             whole(c.out_stride_b, c.out_stride_h, c.out_stride_t)));
+}
+
+template <typename T>
+static void launch_rope_pieces(const uttt_rope_append_args& a, const uttt_kv_roll_args& c, hipStream_t st) {
+  if (a.x != nullptr) {
+    hipLaunchKernelGGL((k_rope_roll<T, true>), dim3((unsigned)a.tokens, (unsigned)a.batch), dim3(kThreads), 0, st, a, c);
+    return;
+  }
+  const int64_t ph = a.head_dim / 2 * sizeof(T) / 16, nv = 2 * ph * a.n_kv_heads;
+  const int64_t n = a.tokens * ((a.n_heads + a.n_kv_heads) * ph + nv) + c.history * 2 * nv;
+  hipLaunchKernelGGL((k_rope_roll<T, false>), dim3((unsigned)((n + kThreads - 1) / kThreads), (unsigned)a.batch),
+                     dim3(kThreads), 0, st, a, c);
+}
+
+extern "C" int uttt_rope_kv_append(const uttt_rope_append_args* a, uttt_stream_t stream) {
+  const int rc = validate_rope(a);
+  if (rc != UTTT_OK) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const uttt_kv_roll_args none{};
   const dim3 grid((unsigned)a->tokens, (unsigned)a->batch);
-  if (a->act_dtype == UTTT_DTYPE_BF16)
+  if (rope_in_pieces(*a, none)) {
+    if (a->act_dtype == UTTT_DTYPE_BF16)
+      launch_rope_pieces<bf16>(*a, none, st);
+    else
+      launch_rope_pieces<float>(*a, none, st);
+  } else if (a->act_dtype == UTTT_DTYPE_BF16) {
     hipLaunchKernelGGL(k_rope_append<bf16>, grid, dim3(kThreads), 0, st, *a);
-  else
+  } else {
     hipLaunchKernelGGL(k_rope_append<float>, grid, dim3(kThreads), 0, st, *a);
+  }
   return launch_status("uttt_rope_kv_append");
+}
+
+extern "C" int uttt_rope_kv_roll(const uttt_rope_append_args* a, const uttt_kv_roll_args* c, uttt_stream_t stream) {
+  const int rc = validate_rope(a);
+  if (rc != UTTT_OK) return rc;
+  UTTT_REQUIRE(c != nullptr, "roll is NULL");
+  UTTT_REQUIRE(a->x == nullptr, "a rolled cache takes no folded norm");
+  UTTT_REQUIRE(c->history >= 0 && c->history <= a->kv_offset && (c->history == 0 || (c->k_hist && c->v_hist)),
+               "history must be in [0, kv_offset] with non-NULL pointers");
+  UTTT_REQUIRE(c->out_len >= 0 && c->out_len <= c->history + a->tokens && (c->out_len == 0 || (c->k_out && c->v_out)),
+               "out_len must be in [0, history + tokens] with non-NULL pointers");
+  UTTT_REQUIRE(rope_in_pieces(*a, *c), "a rolled cache needs 16-byte aligned pointers and strides");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (a->act_dtype == UTTT_DTYPE_BF16)
+    launch_rope_pieces<bf16>(*a, *c, st);
+  else
+    launch_rope_pieces<float>(*a, *c, st);
+  return launch_status("uttt_rope_kv_roll");
 }
 
 extern "C" size_t uttt_swa_prefill_workspace(int64_t batch, int64_t n_heads, int64_t q_len, int64_t kv_len,

@@ -1067,13 +1067,18 @@ def swiglu_readout(x: Tensor, w_up: Tensor, w_gate: Tensor, w_down: Tensor, ln_w
 
 def rope_kv_append(q: Tensor, k: Tensor, v: Tensor, cos: Tensor, sin: Tensor, start_pos: int,
                    k_cache: Tensor, v_cache: Tensor, kv_offset: int, x: Optional[Tensor] = None,
-                   x_eps: float = 0.0, build_only: bool = False):
+                   x_eps: float = 0.0, build_only: bool = False,
+                   history: Optional[Tuple[Tensor, Tensor]] = None, out: Optional[Tuple[Tensor, Tensor]] = None):
     """Rotate ``q`` (B, T, H, hd) in place; write rotated ``k`` and ``v`` (B, T, Hkv, hd) into
     ``k_cache``/``v_cache`` (B, Hkv, L, hd) at time ``kv_offset + t``.  RoPE position of
     token t is ``start_pos + t``; cos/sin are fp32 (positions, hd) tables.  With ``x`` (B, T, D),
     the un-normalised input of a projection whose RMSNorm weight was folded into the weight,
     token t's q / k / v are first scaled by 1 / sqrt(mean(x_t^2) + x_eps).  ``build_only``
-    returns the validated ``uttt_rope_append_args`` without launching."""
+    returns the validated ``uttt_rope_append_args`` without launching.
+
+    ``history`` = (k, v), (B | 1, Hkv, n, hd) each, goes to the caches' rows just before ``kv_offset``;
+    ``out`` = (k, v), (B, Hkv, m, hd) with shared strides, receives the last m rows of history and new
+    ones together: in the same launch where the operands are 16-byte aligned, by copies otherwise."""
     bsz, tokens, heads, hd = q.shape
     hkv = k.shape[2]
     if k.shape != (bsz, tokens, hkv, hd) or v.shape != k.shape:
@@ -1118,8 +1123,65 @@ def rope_kv_append(q: Tensor, k: Tensor, v: Tensor, cos: Tensor, sin: Tensor, st
     if build_only:
         return a
     lib = N.load_library()
+    if history is not None or out is not None:
+        roll = None if x is not None else _kv_roll(a, q, k_cache, history, out)
+        if roll is not None:
+            with torch.cuda.device(dev):
+                N.check(lib.uttt_rope_kv_roll(C.byref(a), C.byref(roll), _stream(dev)), "uttt_rope_kv_roll")
+            return
+        if history is not None:
+            n = history[0].shape[2]
+            k_cache[:, :, kv_offset - n:kv_offset].copy_(history[0])
+            v_cache[:, :, kv_offset - n:kv_offset].copy_(history[1])
     with torch.cuda.device(dev):
         N.check(lib.uttt_rope_kv_append(C.byref(a), _stream(dev)), "uttt_rope_kv_append")
+    if out is not None:
+        end, m = kv_offset + tokens, out[0].shape[2]
+        out[0].copy_(k_cache[:, :, end - m:end])
+        out[1].copy_(v_cache[:, :, end - m:end])
+
+
+def _kv_roll(a: "N.RopeAppendArgs", q: Tensor, k_cache: Tensor, history: Optional[Tuple[Tensor, Tensor]],
+             out: Optional[Tuple[Tensor, Tensor]]) -> Optional["N.KvRollArgs"]:
+    """The cache part of a ``uttt_rope_kv_roll`` call, or None where its operands are not what that
+    call takes (another type or device, rows that are not whole 16-byte pieces)."""
+    vec = 16 // q.element_size()
+    if a.head_dim % (2 * vec):
+        return None
+    c = N.KvRollArgs()
+    groups = [(a.q, a.q_stride_b, a.q_stride_t, a.q_stride_h), (a.k, a.k_stride_b, a.k_stride_t, a.k_stride_h),
+              (a.v, a.v_stride_b, a.v_stride_t, a.v_stride_h),
+              (a.k_cache, a.kv_stride_b, a.kv_stride_h, a.kv_stride_t), (a.v_cache, 0), (a.cos_table, 0),
+              (a.sin_table, 0)]
+    if history is not None:
+        hk, hv = history
+        want = (q.shape[0], k_cache.shape[1], hk.shape[2], k_cache.shape[3])
+        if hk.shape[2] > a.kv_offset:
+            raise ValueError("the history does not fit before kv_offset")
+        for t in (hk, hv):
+            if (t.dtype != q.dtype or t.device != q.device or t.dim() != 4 or t.stride(-1) != 1
+                    or tuple(t.shape[1:]) != want[1:] or t.shape[0] not in (1, want[0])):
+                return None
+        hk, hv = (t.expand(want) for t in (hk, hv))  # one cache for every row, as a copy would broadcast it
+        c.k_hist, c.k_hist_stride_b, c.k_hist_stride_h, c.k_hist_stride_t = _p(hk), *hk.stride()[:3]
+        c.v_hist, c.v_hist_stride_b, c.v_hist_stride_h, c.v_hist_stride_t = _p(hv), *hv.stride()[:3]
+        c.history = hk.shape[2]
+        groups += [(_p(hk), *hk.stride()[:3]), (_p(hv), *hv.stride()[:3])]
+    if out is not None:
+        ok, ov = out
+        for t in (ok, ov):
+            if (t.dtype != q.dtype or t.device != q.device or t.stride() != ok.stride() or t.stride(-1) != 1
+                    or tuple(t.shape) != (q.shape[0], k_cache.shape[1], ok.shape[2], k_cache.shape[3])):
+                return None
+        if ok.shape[2] > c.history + a.tokens:
+            return None
+        c.k_out, c.v_out = _p(ok), _p(ov)
+        c.out_stride_b, c.out_stride_h, c.out_stride_t = ok.stride()[:3]
+        c.out_len = ok.shape[2]
+        groups += [(c.k_out, *ok.stride()[:3]), (c.v_out, 0)]
+    if any(p % 16 or any(st % vec for st in strides) for p, *strides in groups):
+        return None
+    return c
 
 
 # ---------------------------------------------------------------------------

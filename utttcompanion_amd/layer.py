@@ -452,9 +452,11 @@ class SlidingWindowAttention(nn.Module):
         return self._fold
 
     def project(self, x: Tensor, start_pos: int, k_buf: Tensor, v_buf: Tensor, kv_offset: int,
-                norm: Optional["RMSNorm"] = None) -> Tensor:
+                norm: Optional["RMSNorm"] = None, history: Optional[Tuple[Tensor, Tensor]] = None,
+                out: Optional[Tuple[Tensor, Tensor]] = None) -> Tensor:
         """QKV projection + RoPE; writes rotated k / v into the KV buffers at ``kv_offset`` and
-        returns rotated q as a (B, T, H, hd) view.  With ``norm``, ``x`` is the un-normalised
+        returns rotated q as a (B, T, H, hd) view.  ``history`` rows go in front of them and ``out``
+        receives the last rows of both (``kernels.rope_kv_append``).  With ``norm``, ``x`` is the un-normalised
         input of that RMSNorm: its weight is folded into the projection weight and the per-token
         1 / rms scale is applied inside the RoPE kernel, so the norm needs no launch of its own."""
         bsz, seq, _ = x.shape
@@ -464,7 +466,8 @@ class SlidingWindowAttention(nn.Module):
         q, k, v = qkv[:, :, :h], qkv[:, :, h:h + hkv], qkv[:, :, h + hkv:]
         cos, sin = self.rope.tables(start_pos + seq, x.device)
         K.rope_kv_append(q, k, v, cos, sin, start_pos, k_buf, v_buf, kv_offset,
-                         x=None if norm is None else x, x_eps=0.0 if norm is None else norm.eps)
+                         x=None if norm is None else x, x_eps=0.0 if norm is None else norm.eps,
+                         history=history, out=out)
         return q
 
     def forward(self, x: Tensor, kv_cache: Optional[Tuple[Tensor, Tensor]] = None,
@@ -477,19 +480,16 @@ class SlidingWindowAttention(nn.Module):
         hist = 0
         if kv_cache is not None:
             hist = min(kv_cache[0].shape[2], win - 1)
-        k_buf = torch.empty((bsz, hkv, hist + seq, hd), dtype=x.dtype, device=x.device)
+        kv_len = hist + seq
+        k_buf = torch.empty((bsz, hkv, kv_len, hd), dtype=x.dtype, device=x.device)
         v_buf = torch.empty_like(k_buf)
-        if hist:
-            k_buf[:, :, :hist].copy_(kv_cache[0][:, :, -hist:])
-            v_buf[:, :, :hist].copy_(kv_cache[1][:, :, -hist:])
-        q = self.project(x, start_pos, k_buf, v_buf, hist)
+        history = None if not hist else (kv_cache[0][:, :, -hist:], kv_cache[1][:, :, -hist:])
+        cache, trimmed = (k_buf, v_buf), None
+        if kv_len > win:
+            cache = trimmed = tuple(torch.empty((bsz, hkv, win, hd), dtype=x.dtype, device=x.device) for _ in range(2))
+        q = self.project(x, start_pos, k_buf, v_buf, hist, history=history, out=trimmed)
         attn = torch.empty((bsz, seq, self.n_heads, hd), dtype=x.dtype, device=x.device)
         K.swa_prefill(q.transpose(1, 2), k_buf, v_buf, win, hist, out=attn.transpose(1, 2))
-        kv_len = hist + seq
-        if kv_len > win:
-            cache = (k_buf[:, :, -win:].contiguous(), v_buf[:, :, -win:].contiguous())
-        else:
-            cache = (k_buf, v_buf)
         return self.wo(attn.view(bsz, seq, self.d_model)), cache
 
 
