@@ -30,9 +30,11 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 import torch.nn.functional as F
 
+from . import _native as N
 from . import kernels as K
 from .layer import FastWeightState, linear_residual, require_write_chunk
 from .model import PAD_ID, uTTTModel
+from .prefill_plan import PrefillPlan, plan_supported
 
 Tensor = torch.Tensor
 
@@ -56,6 +58,45 @@ def _as_row(t: Tensor, name: str) -> Tensor:
     if t.dim() != 1 or t.shape[0] == 0:
         raise ValueError(f"{name} must be a non-empty (T,) or (1, T) tensor")
     return t
+
+
+def _run_planned(model: uTTTModel, h: Tensor, mask: Tensor, active: Sequence[int], cur: Sequence[Tensor],
+                 copies: Sequence[Tensor], ln_w: Tensor, ln_b: Tensor, k_bufs: Sequence[Tensor],
+                 v_bufs: Sequence[Tensor], surprise: Tensor, row_loss: Tensor, min_chunk_surprise: float, main,
+                 side) -> None:
+    """Every chunk of a bf16 ragged update in one library call each (``uttt_prefill_chunk``), as the
+    model's prefill with writes runs them, over a plan per number of running rows; adds each row's
+    loss sums and token counts to ``row_loss`` (layers, rows, 2).  8 requests of up to 2048 tokens
+    through 4 layers at d 2048: 70.5 -> 69.5 ms a turn against launches one by one."""
+    pool, c, n_layers, dev = model.fast_weight_pool, model.config.chunk_size, len(model.layers), h.device
+    n, seq = mask.shape
+    losses = torch.zeros((len(active), n_layers * n * 2), dtype=torch.float32, device=dev)
+    plan = last = ws = pending = None  # pending: the state-write event of the last chunk enqueued
+    plan_rows = 0
+    try:
+        for ci, rows in enumerate(active):
+            chunk_loss = losses[ci, :n_layers * rows * 2].view(n_layers, rows, 2)
+            if rows != plan_rows:
+                # ``last`` keeps the plan whose state write may still run; the one before it is
+                # done by the time main, which has waited for it, reuses its memory
+                last, plan_rows = plan, rows
+                lead = [t[:rows] for t in copies]
+                run = K.ChunkChainRun(n_layers, c, [t[:rows] for t in cur], ln_w, ln_b, None, pool.momentum_beta,
+                                      float(pool.max_inner_grad_norm or 0.0), pool.normalize_loss_by_dim, pool.eps,
+                                      h.dtype, copies=lead, surprise=surprise[ci], row_loss=chunk_loss,
+                                      min_row_surprise=min_chunk_surprise, workspace=ws, w_products_given=True)
+                ws = run.workspace  # the first plan has the most rows
+                plan = PrefillPlan(model, rows, c, dev, [t[:rows] for t in k_bufs], [t[:rows] for t in v_bufs], seq,
+                                   seq, lead[:3], ln_w, ln_b, pool.eps, run)
+            pending = plan.run(h[:rows], ci * c, ci * c, ci * c, mask[:rows], surprise[ci], main, side,
+                               defer_join=True, wait_event=pending, row_loss=chunk_loss)
+    finally:
+        if pending is not None:
+            N.check(N.load_library().uttt_stream_wait_event(main.cuda_stream, pending), "uttt_stream_wait_event")
+    for rows in sorted(set(active)):  # the chunks that ran this many rows follow each other
+        first = active.index(rows)
+        part = losses[first:first + active.count(rows), :n_layers * rows * 2].sum(0)
+        row_loss[:, :rows] += part.view(n_layers, rows, 2)
 
 
 @torch.no_grad()
@@ -149,7 +190,11 @@ def ragged_test_time_update(model: uTTTModel, interactions: Sequence[Tensor],
     if long_chunks:  # one update per layer; two state sets that swap roles per chunk
         sets = [cur, tuple(torch.empty_like(t) for t in cur)]
         ws_update = None
-    for ci in range(n_chunks):
+    planned = not long_chunks and plan_supported(model, h, copies)
+    if planned:
+        _run_planned(model, h, mask, active, cur, copies, ln_w, ln_b, k_bufs, v_bufs, surprise, row_loss,
+                     min_chunk_surprise, main, side)
+    for ci in range(0 if planned else n_chunks):
         rows, off = active[ci], ci * c
         end = off + c
         cur_mask = mask[:rows, off:end]

@@ -74,9 +74,12 @@ class PrefillPlan:
                    ((n_qkv, dim), (dim, heads * hd), (3 * dim + 2, dim), (dim, dim)))
         self.linear_ws = torch.zeros(max(need, 256), dtype=torch.uint8, device=dev)
         # the attention's split count (and partials) depends on the keys in range: size the
-        # workspace for every KV length a chunk of this plan can see
+        # workspace for every KV length a chunk of this plan can see.  The count follows the number
+        # of 64-key tiles, so lengths 64 apart (and the last) meet each one; a query per length cost
+        # host time that grew with the prompt (8 x 500 tokens, 4 layers: 6.68 -> 6.51 ms a prefill,
+        # 8.53 -> 7.98 ms for a new state's first)
         nbytes = max(lib.uttt_swa_prefill_workspace(bsz, heads, tokens, kv, hd, win)
-                     for kv in range(tokens, kv_capacity + 1))
+                     for kv in [*range(tokens, kv_capacity, 64), kv_capacity])
         self.attn_ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
         self.read_ws = K.readout_workspace(self.hid, read[0])
         hid2 = self.hid.view(rows, dim)
@@ -174,10 +177,12 @@ class PrefillPlan:
 
     def run(self, h: Tensor, off: int, start_pos: int, kv_offset: int, mask: Optional[Tensor],
             surprise: Tensor, main: "torch.cuda.Stream", side: "torch.cuda.Stream", defer_join: bool = False,
-            wait_event: Optional[int] = None) -> Optional[int]:
+            wait_event: Optional[int] = None, row_loss: Optional[Tensor] = None) -> Optional[int]:
         """One chunk: rows ``off .. off + tokens`` of ``h`` (B, T, D) are updated in place through
         every layer, and the chain writes the state; ``mask`` is the fp32 (B, T) token mask (or
-        None) and ``surprise`` this chunk's (layers,) row.  ``defer_join``: ``main`` does not wait
+        None), ``surprise`` this chunk's (layers,) row and ``row_loss`` (optional) the (layers, B, 2)
+        fp32 tensor that receives its per-row loss sums and token counts (given once, a plan's later
+        calls write there too unless they give their own).  ``defer_join``: ``main`` does not wait
         for the state write; the call returns the state write's event handle, which the caller
         passes as ``wait_event`` to its next call (of this plan or another plan of the same
         prefill), whose ``main`` waits for it before its layer-0 readout (consecutive chunks of a
@@ -205,6 +210,11 @@ class PrefillPlan:
         else:
             a.token_mask, a.mask_row_stride = None, 0
         a.surprise = surprise.data_ptr()
+        if row_loss is not None:
+            if (row_loss.shape != (self.n_layers, h.shape[0], 2) or row_loss.dtype != torch.float32
+                    or not row_loss.is_contiguous()):
+                raise ValueError("row_loss must be a contiguous fp32 (layers, B, 2) tensor")
+            a.chain.contents.row_loss = row_loss.data_ptr()  # the call copies the chain's arguments
         lib = N.load_library()
         N.check(lib.uttt_prefill_chunk(C.byref(a), main.cuda_stream, side.cuda_stream), "uttt_prefill_chunk")
         h[:, off:end].copy_(self.hid)
