@@ -18,6 +18,7 @@ CASES = [
     (2, 129, 64, 320, "shared", False, 0.01), # three token blocks
     (1, 300, 256, 192, "own", True, 0.01),    # five
     (8, 37, 320, 256, "shared", True, 1.0),
+    (2, 40, 64, 8256, "own", True, 0.01),     # 129 norm partials, one past the straight loads
 ]
 
 

@@ -19,7 +19,8 @@
 //   4. k_backward / update_mm.hip       dH, dU, dG per F tile + the squared gradient norm partials
 //   5. k_apply / update_mm.hip          recompute each gradient tile from the small activations and
 //                                       apply clip / momentum / decay / inactive-row select to W
-//                                       and S in one pass (bf16: k_row_scalars first)
+//                                       and S in one pass (bf16, several token blocks: k_row_scalars
+//                                       first)
 // Steps 1, 2 and the readout half of 3 alone are the frozen readout.
 #include <algorithm>
 #include <mutex>
@@ -726,8 +727,8 @@ __device__ __forceinline__ void apply_row_scalars(const ApplyArgs& a, int b, flo
   }
 }
 
-// The same scalars once per row (bf16 path): out (B, 4) = clip factor, decay, active flag.  A chunk
-// of several token blocks has a norm partial per gradient tile (2112 at d 1024, F 2816), too many
+// The same scalars once per row (bf16, several token blocks): out (B, 4) = clip factor, decay, active
+// flag.  Such a chunk has a norm partial per gradient tile (2112 at d 1024, F 2816), too many
 // for every workgroup of the apply to sum: that took most of its 147 us at 2 rows of 128 tokens.
 template <typename T>
 __global__ void __launch_bounds__(kThreads) k_row_scalars(const ApplyArgs a, float* out) {
@@ -993,7 +994,15 @@ static void launch_update(const uttt_chunk_update_args& a, char* ws, const Updat
       u.w[i] = ap.w[i]; u.s[i] = ap.s[i]; u.w_out[i] = ap.w_out[i]; u.s_out[i] = ap.s_out[i];
     }
     float* scalars = f.zp;  // the Z partials are consumed by then
-    u.beta = a.momentum_beta; u.nrm = bw.nrm; u.scalars = scalars;
+    u.beta = a.momentum_beta;
+    if (ntb > 1) {
+      u.nrm = bw.nrm; u.scalars = scalars;
+    } else {
+      u.tile_nrm = bw.nrm; u.alpha = a.alpha; u.alpha_rs = a.alpha_row_stride;
+      u.mask = a.token_mask; u.mask_rs = a.mask_row_stride; u.loss = g.loss;
+      u.max_norm = a.max_inner_grad_norm; u.min_row_surprise = a.min_row_surprise;
+      u.surprise = a.surprise; u.row_loss = a.row_loss;
+    }
     if (want(3)) {
       UpdateBackArgs k{};
       k.B = B; k.C = C; k.D = D; k.F = F; k.ntb = ntb; k.tok_pad = TP;
@@ -1004,7 +1013,7 @@ static void launch_update(const uttt_chunk_update_args& a, char* ws, const Updat
       if (ntb > 1 && a.max_inner_grad_norm > 0.f) launch_update_norm(u, st);
     }
     if (want(4)) {
-      hipLaunchKernelGGL(k_row_scalars<T>, dim3(B), blk, 0, st, ap, scalars);
+      if (ntb > 1) hipLaunchKernelGGL(k_row_scalars<T>, dim3(B), blk, 0, st, ap, scalars);
       launch_update_write(u, st);
     }
   } else {

@@ -34,8 +34,20 @@ struct UpdateWriteArgs {
   float* w_out[3];
   float* s_out[3];
   float beta;
-  const float* scalars;  // (B, 4): clip factor, decay, active flag
-  float* nrm;            // norm form: (B, 3 (D / 64) (F / 64)) squared norms of the gradient tiles
+  // several token blocks: the row scalars (B, 4) = clip factor, decay, active flag, and the norm
+  // form's output, (B, 3 (D / 64) (F / 64)) squared norms of the gradient tiles
+  const float* scalars;
+  float* nrm;
+  // one token block: what the write forms the row scalars from (scalars null)
+  const float* tile_nrm;  // (B, F / 64), k_update_back's
+  const void* alpha;      // bf16 (B, C)
+  int64_t alpha_rs;
+  const float* mask;  // (B, C) or null
+  int64_t mask_rs;
+  const float* loss;  // (B, 64)
+  float max_norm, min_row_surprise;
+  float* surprise;
+  float* row_loss;  // (B, 2) or null
 };
 // The squared norm of every gradient tile (more than one token block), and the state write.
 void launch_update_norm(const UpdateWriteArgs& a, hipStream_t st);
