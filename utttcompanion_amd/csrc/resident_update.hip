@@ -9,10 +9,11 @@
 // [v D / 4, (v + 1) D / 4).  Its slice of W_up | W_gate stays in registers, its slices of W_down and
 // of the momentum in LDS, each element at the lane that forms its gradient.
 // Per chunk (C <= 64 tokens; q and k run through the same pre-update W):
-//   1. U | G (64 x 16) for the keys and the queries: every wave over its features, the four
-//      partial sums added in LDS; H = SiLU(G) U
-//   2. the key path's Z partials (H W_down[cols, :])^T over each wave's features -> workspace; the
-//      query path's H and this chunk's W_down[cols, :] saved for the readout;    grid barrier
+//   1. U | G (64 x 16) for the keys: every wave over its features, the four partial sums added in
+//      LDS; H = SiLU(G) U
+//   2. the key path's Z partials (H W_down[cols, :])^T over each wave's features -> workspace;
+//      grid barrier, and between its arrival and its wait the queries' H, which only the readout
+//      needs, and the saves for it (H and this chunk's W_down[cols, :])
 //   3. one key row per workgroup: Z = sum of the partials, LayerNorm, token loss, dZ (stored for
 //      every workgroup);                                                          grid barrier
 //   4. per feature tile of 16: dH partial (dZ W_down^T), (dZ^T H)^T; dH summed over the waves,
@@ -110,12 +111,15 @@ __device__ __forceinline__ void st4_coherent(__amdgpu_buffer_rsrc_t rs, int off,
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rs, off, 0, kCoherent);
 }
 
-// Every workgroup arrives, then waits until all have arrived for the `round`-th time.
-__device__ void grid_barrier(const ResArgs& a, unsigned round) {
+// Every workgroup arrives, then waits until all have arrived for the `round`-th time.  Work that no
+// other workgroup waits for goes between the two.
+__device__ __forceinline__ void grid_arrive(const ResArgs& a) {
   wait_vmcnt<0>();  // this wave's device-coherent stores are complete
   __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_fetch_add(ws_counter(a), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ void grid_wait(const ResArgs& a, unsigned round) {
   if (threadIdx.x == 0) {
-    __hip_atomic_fetch_add(ws_counter(a), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned target = round * gridDim.x;
     if (__hip_atomic_load(ws_flag(a), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) {
       unsigned spins = 0;
@@ -130,6 +134,11 @@ __device__ void grid_barrier(const ResArgs& a, unsigned round) {
     }
   }
   __syncthreads();
+}
+
+__device__ __forceinline__ void grid_barrier(const ResArgs& a, unsigned round) {
+  grid_arrive(a);
+  grid_wait(a, round);
 }
 
 struct OutPtrs {
@@ -305,7 +314,7 @@ __global__ void __launch_bounds__(kThreads, 1) k_resident_update(const ResArgs a
   constexpr int DW = D / 4;      // features per wave: ND tiles of 16
   constexpr int WDLD = D + 4;    // W_down row stride in LDS (spreads the 8 rows over banks)
   __shared__ __align__(16) float wdn[kCols * WDLD];  // W_down [c][d]
-  __shared__ float part_lds[4 * 2 * 64 * kUgLd];      // per-wave U | G partials [v][p][t][c]; dH partials; row sums
+  __shared__ float part_lds[4 * 64 * kUgLd];          // per-wave U | G partials [v][t][c]; dH partials; row sums
   __shared__ __align__(16) float hs[2][64 * kCols];   // H of the keys / queries [t][c]
   __shared__ float uk[64 * kCols], gk[64 * kCols];    // U, G of the keys
   __shared__ __align__(16) float hkt[kCols * kTLd];   // H^T of the keys [c][t]
@@ -347,77 +356,67 @@ __global__ void __launch_bounds__(kThreads, 1) k_resident_update(const ResArgs a
   }
   __syncthreads();
   unsigned round = 0;
-  // step 1 keeps three feature tiles of key and query rows in flight; the first two of a chunk are
+  // the first product keeps three feature tiles of rows in flight; the first two of a chunk's keys are
   // issued at the end of the previous chunk
-  f32x4 xb[3][2][4];
+  f32x4 xb[3][4];
   {
     const int tb = a.c_begin * a.CS, C0 = min(a.CS, a.T - tb);
-    load_rows(a.k + (int64_t)tb * D, D, dbase, C0, col, kq, xb[0][0]);
-    load_rows(a.q + (int64_t)tb * D, D, dbase, C0, col, kq, xb[0][1]);
-    if (ND > 1) {
-      load_rows(a.k + (int64_t)tb * D, D, dbase + 16, C0, col, kq, xb[1][0]);
-      load_rows(a.q + (int64_t)tb * D, D, dbase + 16, C0, col, kq, xb[1][1]);
-    }
+    load_rows(a.k + (int64_t)tb * D, D, dbase, C0, col, kq, xb[0]);
+    if (ND > 1) load_rows(a.k + (int64_t)tb * D, D, dbase + 16, C0, col, kq, xb[1]);
   }
 
   for (int c = a.c_begin; c < a.c_end; ++c) {
     const int t0 = c * a.CS, C = min(a.CS, a.T - t0);
     const float* xk = a.k + (int64_t)t0 * D;
     const float* xq = a.q + (int64_t)t0 * D;
-    // ---------------- 1. U | G partials over this wave's features, both paths
-    {
-      f32x4 acc[2][4];
+    // U | G partials of one path's rows over this wave's features (tiles 0 and 1 in flight), summed
+    // over the waves (in wave order), H = SiLU(G) U
+    auto up_gate = [&](const float* x, bool keys) {
+      f32x4 acc[4];
 #pragma unroll
-      for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[p][r] = zero4();
+      for (int r = 0; r < 4; ++r) acc[r] = zero4();
 #pragma unroll
       for (int m = 0; m < ND; ++m) {
-        if (m + 2 < ND) {
-          load_rows(xk, D, dbase + 16 * (m + 2), C, col, kq, xb[(m + 2) % 3][0]);
-          load_rows(xq, D, dbase + 16 * (m + 2), C, col, kq, xb[(m + 2) % 3][1]);
-        }
+        if (m + 2 < ND) load_rows(x, D, dbase + 16 * (m + 2), C, col, kq, xb[(m + 2) % 3]);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int p = 0; p < 2; ++p)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[p][r] = mfma4(xb[m % 3][p][r][i], w_ug[m][i], acc[p][r]);
+          for (int r = 0; r < 4; ++r) acc[r] = mfma4(xb[m % 3][r][i], w_ug[m][i], acc[r]);
       }
-      // acc[p][r][j] = partial U | G of token 16 r + 4 kq + j, column col
+      // acc[r][j] = partial U | G of token 16 r + 4 kq + j, column col
 #pragma unroll
-      for (int p = 0; p < 2; ++p)
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int j = 0; j < 4; ++j) part_lds[(wave * 64 + 16 * r + 4 * kq + j) * kUgLd + col] = acc[r][j];
+      __syncthreads();
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            part_lds[((wave * 2 + p) * 64 + 16 * r + 4 * kq + j) * kUgLd + col] = acc[p][r][j];
-    }
-    __syncthreads();
-    // U | G summed over the waves (in wave order), H = SiLU(G) U
+      for (int j = 0; j < 2; ++j) {
+        const int e = threadIdx.x + j * kThreads;  // (t, c): 64 x 8
+        const int t = e >> 3, cc = e & 7;
+        float u = 0.f, g = 0.f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int e = threadIdx.x + j * kThreads;  // (p, t, c): 2 x 64 x 8
-      const int p = e >> 9, t = (e >> 3) & 63, cc = e & 7;
-      float u = 0.f, g = 0.f;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const float* row = part_lds + ((v * 2 + p) * 64 + t) * kUgLd;
-        u += row[cc];
-        g += row[cc + kCols];
+        for (int v = 0; v < 4; ++v) {
+          const float* row = part_lds + (v * 64 + t) * kUgLd;
+          u += row[cc];
+          g += row[cc + kCols];
+        }
+        const float h = (g * sigmoidf_acc(g)) * u;
+        hs[keys ? 0 : 1][t * kCols + cc] = h;
+        if (keys) {
+          uk[t * kCols + cc] = u;
+          gk[t * kCols + cc] = g;
+          hkt[cc * kTLd + t] = h;
+        }
       }
-      const float h = (g * sigmoidf_acc(g)) * u;
-      hs[p][t * kCols + cc] = h;
-      if (p == 0) {
-        uk[t * kCols + cc] = u;
-        gk[t * kCols + cc] = g;
-        hkt[cc * kTLd + t] = h;
-      }
-    }
-    __syncthreads();
+      __syncthreads();
+    };
+    // ---------------- 1. the keys' U | G and H
+    up_gate(xk, true);
+    // the queries' first tiles, on their way during the Z partials
+    load_rows(xq, D, dbase, C, col, kq, xb[0]);
+    if (ND > 1) load_rows(xq, D, dbase + 16, C, col, kq, xb[1]);
     // ---------------- 2. the key path's Z^T partials over this wave's features:
-    // (W_down[cols, d])^T H^T; the query path's H and this chunk's W_down[cols, :] are saved for the
-    // readout, which runs after the launch
+    // (W_down[cols, d])^T H^T
     {
       const __amdgpu_buffer_rsrc_t pw = buffer_rsrc(ws_part<D>(a) + (int64_t)w * 64 * D, 64u * D * 4u);
 #pragma unroll
@@ -433,6 +432,14 @@ __global__ void __launch_bounds__(kThreads, 1) k_resident_update(const ResArgs a
           if (t < C) st4_coherent(pw, (t * D + dbase + 16 * n + 4 * kq) * 4, z);
         }
       }
+    }
+    grid_arrive(a);
+    // while the other workgroups arrive: the queries' H, which no workgroup waits for, and it and this
+    // chunk's W_down[cols, :] saved for the readout, which runs after the launch (beside the keys' product
+    // and before the arrival they were on every chunk's critical path: a block of 1024 tokens at d 512,
+    // F 1024 took 911 us, 874 us so)
+    up_gate(xq, false);
+    {
       const int slot = c - a.c_begin;
       if (threadIdx.x < 128) {  // H of the queries: rows t, columns f0 .. f0 + 7
         const int t = threadIdx.x >> 1, half = threadIdx.x & 1;
@@ -448,7 +455,7 @@ __global__ void __launch_bounds__(kThreads, 1) k_resident_update(const ResArgs a
             *reinterpret_cast<const f32x4*>(&wdn[cc * WDLD + 4 * d4]);
       }
     }
-    grid_barrier(a, ++round);
+    grid_wait(a, ++round);
     // ---------------- 3. key rows: Z, LayerNorm, loss and dZ
     for (int t = w; t < C; t += gridDim.x) {
       ln_row<D>(a, t, t0, C, part_lds, red);
@@ -599,14 +606,10 @@ __global__ void __launch_bounds__(kThreads, 1) k_resident_update(const ResArgs a
           if (col < kCols) s_dn[32 * m] = sd;
         }
       }
-      if (c + 1 < a.c_end) {  // the next chunk's first two feature tiles
+      if (c + 1 < a.c_end) {  // the next chunk's first two feature tiles of keys
         const int tn = t0 + a.CS, Cn = min(a.CS, a.T - tn);
-        load_rows(a.k + (int64_t)tn * D, D, dbase, Cn, col, kq, xb[0][0]);
-        load_rows(a.q + (int64_t)tn * D, D, dbase, Cn, col, kq, xb[0][1]);
-        if (ND > 1) {
-          load_rows(a.k + (int64_t)tn * D, D, dbase + 16, Cn, col, kq, xb[1][0]);
-          load_rows(a.q + (int64_t)tn * D, D, dbase + 16, Cn, col, kq, xb[1][1]);
-        }
+        load_rows(a.k + (int64_t)tn * D, D, dbase, Cn, col, kq, xb[0]);
+        if (ND > 1) load_rows(a.k + (int64_t)tn * D, D, dbase + 16, Cn, col, kq, xb[1]);
       }
       __syncthreads();  // W_down updated in LDS before the next chunk reads it
     }
