@@ -1149,10 +1149,10 @@ def _kv_roll(a: "N.RopeAppendArgs", q: Tensor, k_cache: Tensor, history: Optiona
     if a.head_dim % (2 * vec):
         return None
     c = N.KvRollArgs()
-    groups = [(a.q, a.q_stride_b, a.q_stride_t, a.q_stride_h), (a.k, a.k_stride_b, a.k_stride_t, a.k_stride_h),
-              (a.v, a.v_stride_b, a.v_stride_t, a.v_stride_h),
-              (a.k_cache, a.kv_stride_b, a.kv_stride_h, a.kv_stride_t), (a.v_cache, 0), (a.cos_table, 0),
-              (a.sin_table, 0)]
+    # every pointer, and every stride, in one number: a low bit set in any of them is set there
+    at = a.q | a.k | a.v | a.k_cache | a.v_cache | a.cos_table | a.sin_table
+    steps = (a.q_stride_b | a.q_stride_t | a.q_stride_h | a.k_stride_b | a.k_stride_t | a.k_stride_h | a.v_stride_b
+             | a.v_stride_t | a.v_stride_h | a.kv_stride_b | a.kv_stride_h | a.kv_stride_t)
     if history is not None:
         hk, hv = history
         want = (q.shape[0], k_cache.shape[1], hk.shape[2], k_cache.shape[3])
@@ -1162,24 +1162,32 @@ def _kv_roll(a: "N.RopeAppendArgs", q: Tensor, k_cache: Tensor, history: Optiona
             if (t.dtype != q.dtype or t.device != q.device or t.dim() != 4 or t.stride(-1) != 1
                     or tuple(t.shape[1:]) != want[1:] or t.shape[0] not in (1, want[0])):
                 return None
-        hk, hv = (t.expand(want) for t in (hk, hv))  # one cache for every row, as a copy would broadcast it
-        c.k_hist, c.k_hist_stride_b, c.k_hist_stride_h, c.k_hist_stride_t = _p(hk), *hk.stride()[:3]
-        c.v_hist, c.v_hist_stride_b, c.v_hist_stride_h, c.v_hist_stride_t = _p(hv), *hv.stride()[:3]
-        c.history = hk.shape[2]
-        groups += [(_p(hk), *hk.stride()[:3]), (_p(hv), *hv.stride()[:3])]
+        # one cache for every row, as a copy would broadcast it
+        hk, hv = (t if t.shape[0] == want[0] else t.expand(want) for t in (hk, hv))
+        kb, kh, kt, _ = hk.stride()
+        vb, vh, vt, _ = hv.stride()
+        kp, vp = hk.data_ptr(), hv.data_ptr()
+        c.k_hist, c.k_hist_stride_b, c.k_hist_stride_h, c.k_hist_stride_t = kp, kb, kh, kt
+        c.v_hist, c.v_hist_stride_b, c.v_hist_stride_h, c.v_hist_stride_t = vp, vb, vh, vt
+        c.history = want[2]
+        at |= kp | vp
+        steps |= kb | kh | kt | vb | vh | vt
     if out is not None:
         ok, ov = out
         for t in (ok, ov):
             if (t.dtype != q.dtype or t.device != q.device or t.stride() != ok.stride() or t.stride(-1) != 1
                     or tuple(t.shape) != (q.shape[0], k_cache.shape[1], ok.shape[2], k_cache.shape[3])):
                 return None
-        if ok.shape[2] > c.history + a.tokens:
+        m = ok.shape[2]
+        if m > c.history + a.tokens:
             return None
-        c.k_out, c.v_out = _p(ok), _p(ov)
-        c.out_stride_b, c.out_stride_h, c.out_stride_t = ok.stride()[:3]
-        c.out_len = ok.shape[2]
-        groups += [(c.k_out, *ok.stride()[:3]), (c.v_out, 0)]
-    if any(p % 16 or any(st % vec for st in strides) for p, *strides in groups):
+        ob, oh, ot, _ = ok.stride()
+        kp, vp = ok.data_ptr(), ov.data_ptr()
+        c.k_out, c.v_out, c.out_len = kp, vp, m
+        c.out_stride_b, c.out_stride_h, c.out_stride_t = ob, oh, ot
+        at |= kp | vp
+        steps |= ob | oh | ot
+    if at & 15 or steps & (vec - 1):
         return None
     return c
 
