@@ -44,3 +44,34 @@ def test_prefill_attention_matches_float64(case):
     # score and exponent errors, which are far smaller
     bound = 2.0 ** -8 * (ref.abs() + p @ vd.abs())
     assert bool(((got.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("spread", [1.0, 2.0, 4.0])
+@pytest.mark.parametrize("case", [(2, 4, 2, 700, 1300, 64, 512), (1, 8, 2, 1024, 1024, 128, 1024),
+                                  (1, 4, 1, 64, 900, 128, 512)])  # the last one in key splits
+def test_heaviest_weight_of_a_query_is_not_rounded(case, spread):
+    """Scores with a spread of ``spread``, as trained heads have them: the heaviest key of a query weighs
+    1 before the normalisation, so only the other weights are rounded."""
+    from utttcompanion_amd import kernels as K
+    b, h, hkv, tq, tkv, hd, win = case
+    print(f"peaked attention {case} {spread}", flush=True)
+    g = torch.Generator().manual_seed(sum(case))
+    q = (spread * torch.randn(b, tq, h, hd, generator=g)).bfloat16().cuda().transpose(1, 2)
+    k, v = (torch.randn(b, hkv, tkv, hd, generator=g).bfloat16().cuda() for _ in range(2))
+    off = tkv - tq
+    got = K.swa_prefill(q, k, v, win, off).double()
+    kd, vd = (t.double().repeat_interleave(h // hkv, 1) for t in (k, v))
+    d = (torch.arange(tq, device="cuda")[:, None] + off) - torch.arange(tkv, device="cuda")
+    p = (q.double() @ kd.transpose(-1, -2) / hd ** 0.5).masked_fill((d < 0) | (d >= win), float("-inf")).softmax(-1)
+    ref = p @ vd
+    # half an ulp of the output (2^-8 relative at most) and of every weight but the heaviest; 2^-14 for
+    # the fp32 scores (up to about 30, summed over hd products in fp32) and exponents
+    rest = p.masked_fill(p >= p.amax(-1, keepdim=True), 0.0)
+    bound = 2.0 ** -8 * (ref.abs() + rest @ vd.abs()) + 2.0 ** -14 * (p @ vd.abs())
+    assert bool(((got - ref).abs() <= bound).all())
+    # as a whole: the error of weights rounded against the query's own heaviest, and of the rounded output; the
+    # kernel rounds against the heaviest so far, which is as good (a heaviest weight of other than 1, rounded
+    # too, comes to 1.05, 1.2 and 1.2 of it at the three spreads)
+    w = (p / p.amax(-1, keepdim=True))
+    same = ((w.bfloat16().double() @ vd) / w.sum(-1, keepdim=True)).bfloat16().double()
+    assert float((got - ref).norm()) <= 1.03 * float((same - ref).norm())
