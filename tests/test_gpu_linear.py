@@ -73,3 +73,37 @@ def test_linear_refuses_unsupported_operands():
         K.linear(x, w)
     with pytest.raises(ValueError, match="bf16"):
         K.linear(x.float(), w.float())
+
+
+@pytest.mark.parametrize("m, n, k", [(64, 2048, 2048), (192, 768, 768), (100, 512, 1024)])
+def test_linear_adds_its_k_splits_in_order(m, n, k):
+    """Each split's partial is one term of 2^24, 1, 1, .., -2^24: added up in their order the ones vanish
+    (2^24 + 1 rounds to 2^24) and the sum is 0; started from the last one, whose workgroup may well be
+    the one that adds up, it is their number."""
+    from utttcompanion_amd import _native as N
+    from utttcompanion_amd import kernels as K
+    nbytes = N.load_library().uttt_linear_workspace(m, n, k)
+    assert nbytes > 0
+    s = (nbytes - 4 * 16384) // (4 * 64 * 64 * ((m + 63) // 64) * (n // 64))  # after the counters: 64 x 64 fp32 tiles
+    assert s >= 3
+    print(f"linear split order m {m} n {n} k {k} splits {s}", flush=True)
+    x = torch.zeros(m, k, dtype=torch.bfloat16)
+    w = torch.zeros(n, k, dtype=torch.bfloat16)
+    for i in range(s):
+        first = 64 * (i * (k // 64) // s)  # split i's first column
+        x[:, first] = 1.0
+        w[:, first] = 2.0 ** 24 if i == 0 else -2.0 ** 24 if i == s - 1 else 1.0
+    x, w = x.to(DEV), w.to(DEV)
+    for _ in range(20):
+        assert not bool(K.linear(x, w).any())
+
+
+@pytest.mark.parametrize("m, n, k", [(64, 2048, 2048), (448, 768, 768)])
+def test_linear_repeats_itself(m, n, k):
+    from utttcompanion_amd import kernels as K
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn(m, k, generator=g).bfloat16().to(DEV)
+    w = torch.randn(n, k, generator=g).bfloat16().to(DEV)
+    first = K.linear(x, w)
+    for _ in range(20):
+        assert torch.equal(K.linear(x, w), first)

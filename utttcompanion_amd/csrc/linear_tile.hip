@@ -13,7 +13,7 @@
 // tile.  The launch plan spreads that traffic over the CUs: tiles of MT x 64 (MT 128 or 64) and,
 // when the tiles alone leave CUs idle, a split of the k loop over `splits` workgroups per tile,
 // whose fp32 partial tiles meet in the workspace; the last workgroup of a tile to finish (a
-// counter per tile) adds the others' partials to its own and writes the output.  The kernel
+// counter per tile) adds them up in their order and writes the output.  The kernel
 // times match the library GEMM's at these shapes within about 15% either way; its point is
 // that a native caller can launch it without a library call's host cost.
 //
@@ -147,7 +147,8 @@ __global__ void __launch_bounds__(kLinThreads, 1) k_linear(const LinArgs a) {
   const bool holds = w < NWA;  // this wave holds a distinct block of the tile
   if (a.splits > 1) {
     // store this split's partial tile ([wave][i][lane]) device-coherently, then count; the
-    // workgroup that completes the count adds the other splits' partials (read past its L2)
+    // workgroup that completes the count adds up all splits' partials (the others' read past its
+    // L2), in the order of the splits whichever of them came last, so that equal inputs give equal bits
     constexpr int TILE = MT * NT;
     float* mine = a.part + ((int64_t)tile * a.splits + split) * TILE;
     if (holds) {
@@ -167,8 +168,18 @@ __global__ void __launch_bounds__(kLinThreads, 1) k_linear(const LinArgs a) {
     if (!last) return;
     if (holds) {
       const float* base = a.part + (int64_t)tile * a.splits * TILE + (w * 16) * 64 + lane;
+      float own[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        own[i] = acc[i];
+        acc[i] = 0.f;
+      }
       for (int s = 0; s < a.splits; ++s) {
-        if (s == split) continue;
+        if (s == split) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[i] += own[i];
+          continue;
+        }
         float v[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i)
