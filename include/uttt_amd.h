@@ -370,7 +370,7 @@ typedef struct {
   int64_t batch, n_heads, n_kv_heads, q_len, kv_len, head_dim; /* head_dim 64 or 128 */
   int64_t q_offset, window;
   int32_t act_dtype; /* bf16 or fp32 */
-  float scale;
+  float scale; /* of the scores before the softmax: any value, 1 / sqrt(head_dim) in the model */
   const void* q; int64_t q_stride_b, q_stride_h, q_stride_t;
   const void* k; int64_t k_stride_b, k_stride_h, k_stride_t;
   const void* v; int64_t v_stride_b, v_stride_h, v_stride_t;

@@ -75,3 +75,33 @@ def test_heaviest_weight_of_a_query_is_not_rounded(case, spread):
     w = (p / p.amax(-1, keepdim=True))
     same = ((w.bfloat16().double() @ vd) / w.sum(-1, keepdim=True)).bfloat16().double()
     assert float((got - ref).norm()) <= 1.03 * float((same - ref).norm())
+
+
+@pytest.mark.parametrize("scale", [-0.125, 0.0, 0.3])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("case", [(2, 4, 2, 100, 163, 64, 65), (1, 2, 1, 64, 600, 128, 512)])  # the latter in splits
+def test_any_softmax_scale(case, dtype, scale):
+    """The C entry's ``scale`` may be any number, whatever the type: none, or one that turns the order of
+    the scores round."""
+    import ctypes as C
+    from utttcompanion_amd import _native as N
+    from utttcompanion_amd import kernels as K
+    b, h, hkv, tq, tkv, hd, win = case
+    print(f"attention scale {case} {dtype} {scale}", flush=True)
+    g = torch.Generator().manual_seed(sum(case))
+    q = torch.randn(b, h, tq, hd, generator=g).to(dtype).cuda()
+    k, v = (torch.randn(b, hkv, tkv, hd, generator=g).to(dtype).cuda() for _ in range(2))
+    out = torch.empty_like(q)
+    off = tkv - tq
+    lib = N.load_library()
+    ws = torch.empty(lib.uttt_swa_prefill_workspace(b, h, tq, tkv, hd, win), dtype=torch.uint8, device="cuda")
+    a = K.swa_prefill(q, k, v, win, off, out=out, workspace=ws, build_only=True)
+    a.scale = scale
+    N.check(lib.uttt_swa_prefill(C.byref(a), torch.cuda.current_stream().cuda_stream), "uttt_swa_prefill")
+    kd, vd = (t.double().repeat_interleave(h // hkv, 1) for t in (k, v))
+    d = (torch.arange(tq, device="cuda")[:, None] + off) - torch.arange(tkv, device="cuda")
+    p = (scale * (q.double() @ kd.transpose(-1, -2))).masked_fill((d < 0) | (d >= win), float("-inf")).softmax(-1)
+    ref = p @ vd
+    # bf16: half an ulp (2^-8 relative at most) of the output and of each weight; fp32: sums of up to 600 terms
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -14
+    assert bool(((out.double() - ref).abs() <= unit * (ref.abs() + 1.1 * (p @ vd.abs()))).all())

@@ -28,6 +28,8 @@
 // 28.9 -> 17.9 us; one 64-token chunk of 4 rows over 1088 keys, head_dim 128: 26.2 -> 21.5 us.
 #include "swa_prefill.h"
 
+#include <math.h>
+
 #include <algorithm>
 
 #include "uttt_device.h"
@@ -42,7 +44,7 @@ struct SwaMmArgs {
   int q_len, nqb, wgs;  // 32-query blocks, workgroups per (row, kv head) and split
   int nsplit, tiles_per_split, q_pad, groups;
   int64_t q_offset, kv_len, window;
-  float scale;
+  float scale, q_sign;  // scale > 0; Q enters times q_sign
   const bf16 *q, *k, *v;
   int64_t q_sb, q_sh, q_st, k_sb, k_sh, k_st, v_sb, v_sh, v_st;
   bf16* out;
@@ -145,6 +147,12 @@ __global__ void __launch_bounds__(NW * 64, NW >= 6 ? 1 : 2) k_swa_prefill_mm(con
         qf[s] = *reinterpret_cast<const bf16x8*>(qr + 16 * s);
       else
         qf[s] = bf16x8{};
+    }
+    if (a.q_sign != 1.f) {
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qf[s][e] = from_f32<bf16>(to_f32((bf16)qf[s][e]) * a.q_sign);
     }
   }
 
@@ -397,7 +405,11 @@ void launch_swa_prefill_mm(const uttt_swa_prefill_args& a, float* part, int q_pa
   m.q_len = (int)a.q_len; m.nqb = (int)((a.q_len + kQB - 1) / kQB); m.wgs = p.wgs;
   m.nsplit = p.nsplit; m.tiles_per_split = p.tiles_per_split; m.q_pad = q_pad;
   m.groups = (int)(a.batch * a.n_kv_heads);
-  m.q_offset = a.q_offset; m.kv_len = a.kv_len; m.window = a.window; m.scale = a.scale;
+  m.q_offset = a.q_offset; m.kv_len = a.kv_len; m.window = a.window;
+  // the kernel takes maxima of, and masks, the raw scores, which holds for a positive scale: Q carries
+  // the sign of another one (exact in bf16), and for 0 the scores are 0 whatever their scale
+  m.scale = a.scale != 0.f ? fabsf(a.scale) : 1.f;
+  m.q_sign = a.scale > 0.f ? 1.f : a.scale < 0.f ? -1.f : 0.f;
   m.q = static_cast<const bf16*>(a.q); m.k = static_cast<const bf16*>(a.k); m.v = static_cast<const bf16*>(a.v);
   m.q_sb = a.q_stride_b; m.q_sh = a.q_stride_h; m.q_st = a.q_stride_t;
   m.k_sb = a.k_stride_b; m.k_sh = a.k_stride_h; m.k_st = a.k_stride_t;
