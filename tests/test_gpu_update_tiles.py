@@ -74,3 +74,38 @@ def test_update_matches_float64(case, out):
     bound = 2.0 ** -8 * ref[0].abs() + 7 * 2.0 ** -9 / 3 ** 0.5 * 2.0
     assert bool(((res[0].double().cpu() - ref[0]).abs() <= bound).all())
     assert abs(float(res[7]) - float(ref[7])) <= 2.0 ** -8 * abs(float(ref[7]))
+
+
+@pytest.mark.parametrize("tokens", [37, 64, 129])
+@pytest.mark.parametrize("noise", [1.0, 0.1, 0.01, 0.0])
+def test_clip_factor_of_similar_tokens(tokens, noise):
+    """The applied clip factor against the norm of the gradient itself, read back from an update without
+    clipping (S' = -g from S = 0), where a chunk's keys are nearly one token and their errors nearly cancel:
+    the norm is then a small difference of large sums unless its terms are squares."""
+    from utttcompanion_amd import kernels as K
+    b, d, f, eps = 2, 320, 256, 1e-5
+    print(f"clip factor {tokens} tokens, noise {noise}", flush=True)
+    g = torch.Generator().manual_seed(tokens)
+    k = torch.nn.functional.rms_norm(torch.randn(b, 1, d, generator=g) + noise * torch.randn(b, tokens, d, generator=g),
+                                     (d,)).bfloat16()
+    w = [torch.randn(b, d, f, generator=g) / d ** 0.5, torch.randn(b, d, f, generator=g) / d ** 0.5,
+         torch.randn(b, f, d, generator=g) / f ** 0.5]
+    ln = [1 + 0.1 * torch.randn(d, generator=g), 0.1 * torch.randn(d, generator=g)]
+    kd, w16 = k.double(), [t.bfloat16().double() for t in w]
+    z = (torch.nn.functional.silu(kd @ w16[1]) * (kd @ w16[0])) @ w16[2]
+    sign = torch.tensor([1.0, -1.0]).repeat(tokens)[:tokens] * (1.0 if tokens % 2 == 0 else (torch.arange(tokens) > 0))
+    v = (kd + torch.nn.functional.layer_norm(z, (d,), ln[0].double(), ln[1].double(), eps)
+         + sign[None, :, None] * torch.randn(b, 1, d, generator=g)).bfloat16()
+    eta = torch.full((b, tokens, 1), 0.5).bfloat16()
+    args = [t.cuda() for t in (k, k, v, eta, torch.zeros_like(eta), *w, *(torch.zeros_like(t) for t in w), *ln)]
+    grad = [t.double() for t in K.chunk_update(*args, None, 0.9, 0.0, False, eps)[4:7]]
+    n2 = sum(t.square().sum((1, 2)) for t in grad)
+    clip = 0.25 * float(n2.min().sqrt())
+    got = [t.double() for t in K.chunk_update(*args, None, 0.9, clip, False, eps)[4:7]]
+    # the least squares factor between the two, a mean over their 2^-24 roundings
+    factor = sum((a * t).sum((1, 2)) for a, t in zip(got, grad)) / n2
+    want = clip / (n2 + 1e-8).sqrt()
+    print(n2.tolist(), (factor / want - 1).tolist(), flush=True)
+    # squares added up in fp32 in chains of at most 12 D / 64 + 20 additions, 2^-24 each; half of it in the
+    # root, whose own rounding and the division's are 2^-23
+    assert float((factor / want - 1).abs().max()) <= (12 * d / 64 + 20) * 2.0 ** -25 + 2.0 ** -22

@@ -46,19 +46,45 @@ __device__ __forceinline__ void mma4(f32x16& acc, const bf16x8 (&a)[4], const bf
   for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s], b[s], acc, 0, 0, 0);
 }
 
-// One (F tile, row, token block).  NORM (one token block): the tile's squared gradient norm from
-// Gram matrices, |K^T dU|^2 = <K K^T, dU dU^T> (and alike for dG; |H^T dZ|^2 = <H H^T, dZ dZ^T>):
-// K K^T and dZ dZ^T accumulate over D beside dH from the tiles dH needs anyway, where forming the
-// gradient tiles took a second loop over D with three products and transposes per step.  Sums of
-// 64 x 64 products of fp32 accumulations; the clip factor's relative error stays near 1e-6.
+// the eight transposing reads of a slab's fragments; slab_join after the wait makes the operands of them
+__device__ __forceinline__ void slab_read(uint32_t addr, i16x4 (&r)[8]) {
+  r[0] = lds_read_tr16<0>(addr);
+  r[1] = lds_read_tr16<512>(addr);
+  r[2] = lds_read_tr16<2048>(addr);
+  r[3] = lds_read_tr16<2560>(addr);
+  r[4] = lds_read_tr16<4096>(addr);
+  r[5] = lds_read_tr16<4608>(addr);
+  r[6] = lds_read_tr16<6144>(addr);
+  r[7] = lds_read_tr16<6656>(addr);
+}
+template <int AHEAD>
+__device__ __forceinline__ void slab_wait(i16x4 (&r)[8]) {
+  asm volatile("s_waitcnt lgkmcnt(%8)"
+               : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]), "+v"(r[6]), "+v"(r[7])
+               : "n"(AHEAD));
+}
+__device__ __forceinline__ void slab_join(const i16x4 (&r)[8], bf16x8 (&f)[4]) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    f[k] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(r[2 * k], r[2 * k + 1], 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+__device__ __forceinline__ void lds_write_b16(uint32_t addr, bf16 v) {
+  asm volatile("ds_write_b16 %0, %1" ::"v"(addr), "v"((uint32_t)__builtin_bit_cast(uint16_t, v)));
+}
+
+// One (F tile, row, token block).  NORM (one token block): then the tile's squared gradient norm, the
+// sum of the squares of the gradient tiles K^T dU, K^T dG and dZ^T H, 64 x 64 each, in a second loop
+// over D whose first slabs arrive while dU and dG are formed.  (Gram matrices, <K K^T, dU dU^T> and
+// alike, need no second loop, but their terms have both signs: 1e-6 relative on independent tokens,
+// 1e-2 and more once a chunk's keys are nearly one token.)
 template <bool NORM>
 __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArgs a) {
-  constexpr int TILES = NORM ? 2 : 1;        // dZ rows (and K rows) by direct loads
-  constexpr int SLOT = (TILES + 1) * 8192;   // then the W_down rows, rounded through registers
-  constexpr int PER = TILES * 2, WCH = 4;    // loads per wave and step, W_down pieces per thread
+  constexpr int SLOT = 2 * 8192;      // dZ rows by direct loads, W_down rows rounded through registers
+  constexpr int PER = 2, WCH = 4;     // loads per wave and step, W_down pieces per thread
   constexpr int SLOTS = 3;
   __shared__ __align__(1024) char ring[SLOTS * SLOT];
-  __shared__ __align__(1024) char htile[NORM ? 8192 : 16];
+  __shared__ __align__(1024) char slabs[NORM ? 3 * 8192 : 16];  // token slabs of H, dU, dG
   const int nF = a.F / 64;
   const RowTile rt = row_tile(blockIdx.x, a.B, nF * a.ntb);
   if (!rt.valid) return;
@@ -66,25 +92,19 @@ __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArg
   const int w = uniform((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int wr = (w >> 1) * 32, wc = (w & 1) * 32;
   const bf16* dz = static_cast<const bf16*>(a.dz) + ((int64_t)b * a.tok_pad + t0) * a.D;
-  const bf16* kr = static_cast<const bf16*>(a.k) + (int64_t)b * a.k_rs + (int64_t)t0 * a.D;
   const float* wd = a.w_down + (int64_t)b * a.D * a.F + (int64_t)f0 * a.D;
   const int64_t rowbase = ((int64_t)b * a.tok_pad + t0) * a.F + f0;
-  const uint32_t ring0 = lds_addr(ring), h0 = lds_addr(htile);
-  const uint32_t k_bytes = (uint32_t)uniform(max(0, min(64, a.C - t0)) * a.D * 2);
+  const uint32_t ring0 = lds_addr(ring), slab0 = lds_addr(slabs);
 
   int voff[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) voff[i] = row_src_off(w + 4 * i, lane, a.D);
   auto issue = [&](int step, int at) {
     const uint32_t base = ring0 + (uint32_t)((at % SLOTS) * SLOT);
-    const __amdgpu_buffer_rsrc_t rz = buffer_rsrc(dz + step * 64, (uint32_t)(64 * a.D * 2));
-    const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(kr + step * 64, k_bytes);  // rows past C read as zeros
+    const __amdgpu_buffer_rsrc_t rz = buffer_rsrc(dz + step * 64, (uint32_t)((64 * a.D - step * 64) * 2));
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < 2; ++i)
       buffer_load_lds_raw(rz, lds_ptr(base + (uint32_t)((w + 4 * i) * 1024)), 16, voff[i], 0, 0, 0);
-      if constexpr (NORM)
-        buffer_load_lds_raw(rk, lds_ptr(base + 8192u + (uint32_t)((w + 4 * i) * 1024)), 16, voff[i], 0, 0, 0);
-    }
   };
   // W_down rows: thread's piece i is row 16 i + tid / 16, columns 4 (tid % 16) .. + 3
   struct Pieces {
@@ -93,7 +113,7 @@ __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArg
   const int wrow = (int)threadIdx.x >> 4, wc4 = threadIdx.x & 15;
   const int wsrc = (wrow * a.D + 4 * wc4) * 4;
   const uint32_t wdst =
-      ring0 + (uint32_t)(TILES * 8192 + wrow * 128 + (((wc4 >> 1) ^ row_swz(wrow)) * 16) + (wc4 & 1) * 8);
+      ring0 + (uint32_t)(8192 + wrow * 128 + (((wc4 >> 1) ^ row_swz(wrow)) * 16) + (wc4 & 1) * 8);
   auto wload = [&](Pieces& p, int step) {
     const __amdgpu_buffer_rsrc_t r = buffer_rsrc(wd + step * 64, (uint32_t)(64 * a.D - step * 64) * 4u);
 #pragma unroll
@@ -111,11 +131,11 @@ __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArg
 
   if constexpr (NORM) {
     const __amdgpu_buffer_rsrc_t rh =
-        buffer_rsrc(static_cast<const bf16*>(a.h) + rowbase, (uint32_t)(64 * a.F * 2));
+        buffer_rsrc(static_cast<const bf16*>(a.h) + rowbase, (uint32_t)((64 * a.F - f0) * 2));
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      buffer_load_lds_raw(rh, lds_ptr(h0 + (uint32_t)((w + 4 * i) * 1024)), 16, row_src_off(w + 4 * i, lane, a.F), 0,
-                          0, 0);
+      buffer_load_lds_raw(rh, lds_ptr(slab0 + (uint32_t)((w + 4 * i) * 1024)), 16, slab_src_off(w + 4 * i, lane, a.F),
+                          0, 0, 0);
   }
   const int nsteps = a.D / 64, last = nsteps - 1;
   Pieces p0, p1;
@@ -124,10 +144,8 @@ __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArg
   wload(p1, min(1, last));
   issue(min(1, last), 1);
   wstore(p0, 0);
-  f32x16 dh, zz, kk;
+  f32x16 dh;
   zero(dh);
-  zero(zz);
-  zero(kk);
   // loads run two steps ahead (the last steps load the last step again, so that every iteration has
   // the same loads in flight); a step's W_down pieces reach LDS during the step before it
   auto body = [&](int step, Pieces& mine, Pieces& next) {
@@ -139,20 +157,10 @@ __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArg
     const uint32_t so = ring0 + (uint32_t)((step % SLOTS) * SLOT);
     bf16x8 fa[4], fb[4];
     row_frags(so, wr, lane, fa);
-    row_frags(so + TILES * 8192u, wc, lane, fb);
+    row_frags(so + 8192u, wc, lane, fb);
     wait_frags<4>(fa);
     wait_frags<0>(fb);
     mma4(dh, fa, fb);
-    if constexpr (NORM) {
-      row_frags(so, wc, lane, fb);
-      wait_frags<0>(fb);
-      mma4(zz, fa, fb);
-      row_frags(so + 8192u, wr, lane, fa);
-      row_frags(so + 8192u, wc, lane, fb);
-      wait_frags<4>(fa);
-      wait_frags<0>(fb);
-      mma4(kk, fa, fb);
-    }
     __builtin_amdgcn_sched_barrier(0);
     wstore(next, step + 1);
   };
@@ -162,8 +170,6 @@ __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArg
     body(step + 1, p1, p0);
   }
   if (step < nsteps) body(step, p0, p1);
-  wait_vmcnt<0>();
-  asm volatile("s_waitcnt lgkmcnt(0)");
   float uv[16], gv[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
@@ -171,10 +177,26 @@ __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArg
     uv[i] = a.u[off];
     gv[i] = a.g[off];
   }
-  __syncthreads();  // the ring is free: dU and dG row tiles go to its first two tiles
-
-  bf16* dus = reinterpret_cast<bf16*>(ring);
-  bf16* dgs = reinterpret_cast<bf16*>(ring + 8192);
+  // the second loop's slabs: K, then dZ columns 64 step .. of the block's tokens
+  auto issue_slabs = [&](int step) {
+    const uint32_t base = ring0 + (uint32_t)((step % SLOTS) * SLOT);
+    const bf16* kr = static_cast<const bf16*>(a.k) + (int64_t)b * a.k_rs + step * 64;
+    // token rows past C read as zeros
+    const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(kr, (uint32_t)uniform((a.C * a.D - step * 64) * 2));
+    const __amdgpu_buffer_rsrc_t rz = buffer_rsrc(dz + step * 64, (uint32_t)((64 * a.D - step * 64) * 2));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int off = slab_src_off(w + 4 * i, lane, a.D);
+      buffer_load_lds_raw(rk, lds_ptr(base + (uint32_t)((w + 4 * i) * 1024)), 16, off, 0, 0, 0);
+      buffer_load_lds_raw(rz, lds_ptr(base + 8192u + (uint32_t)((w + 4 * i) * 1024)), 16, off, 0, 0, 0);
+    }
+  };
+  if constexpr (NORM) {
+    wait_vmcnt<0>();  // the repeated loads
+    asm volatile("s_waitcnt lgkmcnt(0)");
+    __builtin_amdgcn_s_barrier();  // the ring is free
+    for (int j = 0; j < min(nsteps, SLOTS - 1); ++j) issue_slabs(j);
+  }
   const int f = wc + acc_col();
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
@@ -186,38 +208,56 @@ __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArg
     static_cast<bf16*>(a.du)[off] = du;
     static_cast<bf16*>(a.dg)[off] = dg;
     if constexpr (NORM) {
-      const int at = t * 64 + (((f >> 3) ^ row_swz(t)) * 8) + (f & 7);
-      dus[at] = du;
-      dgs[at] = dg;
+      const uint32_t at = slab0 + (uint32_t)(t * 128 + (((f >> 3) ^ slab_swz(t)) * 16) + (f & 7) * 2);
+      lds_write_b16(at + 8192u, du);
+      lds_write_b16(at + 16384u, dg);
     }
   }
   if constexpr (NORM) {
-    __syncthreads();
-    f32x16 g1, g2;
-    zero(g1);
-    zero(g2);
-    bf16x8 fa[4], fb[4];
-    row_frags(ring0, wr, lane, fa);
-    row_frags(ring0, wc, lane, fb);
-    wait_frags<4>(fa);
-    wait_frags<0>(fb);
-    mma4(g1, fa, fb);
-    row_frags(ring0 + 8192u, wr, lane, fa);
-    row_frags(ring0 + 8192u, wc, lane, fb);
-    wait_frags<4>(fa);
-    wait_frags<0>(fb);
-    mma4(g1, fa, fb);
-    row_frags(h0, wr, lane, fa);
-    row_frags(h0, wc, lane, fb);
-    wait_frags<4>(fa);
-    wait_frags<0>(fb);
-    mma4(g2, fa, fb);
-    float sq = 0.f;
+    asm volatile("s_waitcnt lgkmcnt(0)");
+    __builtin_amdgcn_s_barrier();  // dU, dG and H slabs are whole
+    bf16x8 bu[4], bg[4], bh[4];
+    {
+      i16x4 ru[8], rg[8], rh[8];
+      slab_read(slab_tr_addr(slab0 + 8192u, wc, lane), ru);
+      slab_wait<0>(ru);
+      slab_join(ru, bu);
+      slab_read(slab_tr_addr(slab0 + 16384u, wc, lane), rg);
+      slab_wait<0>(rg);
+      slab_join(rg, bg);
+      slab_read(slab_tr_addr(slab0, wc, lane), rh);
+      slab_wait<0>(rh);
+      slab_join(rh, bh);
+    }
+    const uint32_t tk = slab_tr_addr(ring0, wr, lane);
+    float sq[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int step = 0; step < nsteps; ++step) {
+      wait_steps<4, SLOTS - 2>(min(nsteps - 1, step + SLOTS - 2) - step);
+      __builtin_amdgcn_s_barrier();  // the step's slabs are in LDS; the oldest slot is free
+      if (step + SLOTS - 1 < nsteps) issue_slabs(step + SLOTS - 1);
+      const uint32_t so = (uint32_t)((step % SLOTS) * SLOT);
+      i16x4 rk[8], rz[8];
+      slab_read(tk + so, rk);
+      slab_read(tk + so + 8192u, rz);
+      bf16x8 fk[4], fz[4];
+      f32x16 gu, gg, gd;
+      zero(gu);
+      zero(gg);
+      zero(gd);
+      slab_wait<8>(rk);
+      slab_join(rk, fk);
+      mma4(gu, fk, bu);
+      mma4(gg, fk, bg);
+      slab_wait<0>(rz);
+      slab_join(rz, fz);
+      mma4(gd, fz, bh);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) sq += kk[i] * g1[i] + zz[i] * g2[i];
-    // the scratch of the sum: the ring past the two tiles (160 KB of LDS hold two workgroups)
-    const float total = block_sum(sq, reinterpret_cast<float*>(ring + 16384));
+      for (int i = 0; i < 16; ++i) sq[i & 3] += gu[i] * gu[i] + gg[i] * gg[i] + gd[i] * gd[i];
+    }
+    const float total = block_sum((sq[0] + sq[1]) + (sq[2] + sq[3]), reinterpret_cast<float*>(ring));
     if (threadIdx.x == 0) a.nrm[b * nF + ft] = total;
+  } else {
+    wait_vmcnt<0>();  // the repeated loads
   }
 }
 
