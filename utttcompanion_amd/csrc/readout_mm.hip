@@ -271,9 +271,11 @@ __global__ void __launch_bounds__(WM* WN * 64) k_readout_mm(const MmArgs a) {
     WPieces p0, p1;
     wload(p0, 0);
     issue(0);
+    pin_loads();
     if constexpr (AHEAD == 2) {
       wload(p1, min(1, last));
       issue_at(min(1, last), 1);
+      pin_loads();
     }
     wstore(p0, 0);
     // the loads of step + AHEAD into `mine` (the pieces of `step`, stored already), then the
@@ -284,6 +286,7 @@ __global__ void __launch_bounds__(WM* WN * 64) k_readout_mm(const MmArgs a) {
       __builtin_amdgcn_s_barrier();
       wload(mine, min(step + AHEAD, last));
       issue_at(min(step + AHEAD, last), step + AHEAD);
+      pin_loads();
       consume(step);
       __builtin_amdgcn_sched_barrier(0);  // no wait for the next pieces before the products are issued
       wstore(next, step + 1);

@@ -141,8 +141,10 @@ __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArg
   Pieces p0, p1;
   wload(p0, 0);
   issue(0, 0);
+  pin_loads();
   wload(p1, min(1, last));
   issue(min(1, last), 1);
+  pin_loads();
   wstore(p0, 0);
   f32x16 dh;
   zero(dh);
@@ -154,6 +156,7 @@ __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArg
     __builtin_amdgcn_s_barrier();
     wload(mine, min(step + 2, last));
     issue(min(step + 2, last), step + 2);
+    pin_loads();
     const uint32_t so = ring0 + (uint32_t)((step % SLOTS) * SLOT);
     bf16x8 fa[4], fb[4];
     row_frags(so, wr, lane, fa);
@@ -357,14 +360,20 @@ __global__ void __launch_bounds__(kThreads) k_update_write(const UpdateWriteArgs
           buffer_rsrc(static_cast<const bf16*>(a.alpha) + (int64_t)b * a.alpha_rs, (uint32_t)a.C * 2u), 2 * lane, 0, 0);
     }
   }
+  float clip = 0.f, decay = 0.f, act = 0.f;
+  if constexpr (FORM == kScalarsGiven) {
+    clip = a.scalars[4 * b];
+    decay = a.scalars[4 * b + 1];
+    act = a.scalars[4 * b + 2];
+  }
   issue(0);
   if (a.ntb > 1) issue(1);
+  pin_loads();
   // the state tile is the bulk of the traffic: its loads go out before the products
   const int64_t mat = (int64_t)a.D * a.F;
   const int row = (int)threadIdx.x >> 4, c4 = threadIdx.x & 15;
   const int64_t at = (int64_t)b * mat + (int64_t)(r0 + row) * ld_out + c0 + 4 * c4;
   f32x4 wv[4], sv[4];
-  float clip = 0.f, decay = 0.f, act = 0.f;
   if constexpr (!NORM) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -372,11 +381,7 @@ __global__ void __launch_bounds__(kThreads) k_update_write(const UpdateWriteArgs
       sv[i] = *reinterpret_cast<const f32x4*>(a.s[m] + at + (int64_t)16 * i * ld_out);
     }
   }
-  if constexpr (FORM == kScalarsGiven) {
-    clip = a.scalars[4 * b];
-    decay = a.scalars[4 * b + 1];
-    act = a.scalars[4 * b + 2];
-  }
+  pin_loads();  // eight of them for the first wait below
   if constexpr (FORM == kFormScalars) {
     if (w == 0) {
       float sq = nrm0 + nrm1;

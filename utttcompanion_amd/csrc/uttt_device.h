@@ -341,6 +341,11 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
+// No load or store of the compiler's own placing moves across it.  A wait that counts such loads
+// (wait_vmcnt<N> with N register loads younger than the direct-to-LDS loads it waits for) is right
+// only while they stay between those loads and the wait: the wait itself holds them back from neither.
+__device__ __forceinline__ void pin_loads() { asm volatile("" ::: "memory"); }
+
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 
 // ds_read_b64_tr_b16: in each group of 16 lanes, lane i receives element (i & 3) of the 8 bytes
