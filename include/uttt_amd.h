@@ -32,7 +32,7 @@ enum { UTTT_OK = 0, UTTT_ERR_INVALID = 1, UTTT_ERR_HIP = 2, UTTT_ERR_WORKSPACE =
 
 /* ABI version of the structures and entry points below: uttt_abi_version() returns it, and the
  * Python binding reads it from this header and refuses a library built from another one. */
-#define UTTT_ABI_VERSION 24
+#define UTTT_ABI_VERSION 25
 
 /* Text of the last error on this host thread ("" when none). */
 const char* uttt_last_error(void);
@@ -347,8 +347,9 @@ int uttt_rope_kv_append(const uttt_rope_append_args* args, uttt_stream_t stream)
 /* The same with a bounded cache around the call (model/uttt_layer.py:1082-1114), in one launch: the
  * last `history` rows of an earlier cache go to [kv_offset - history, kv_offset) of k_cache / v_cache,
  * and rows [kv_offset + tokens - out_len, kv_offset + tokens) of them (history rows first) also go to
- * k_out / v_out.  Both optional (history 0, out_len 0).  Needs 16-byte aligned pointers and strides in
- * whole 16-byte pieces, head_dim a multiple of 16 (bf16) or 8 (fp32), and no folded norm. */
+ * k_out / v_out.  Both optional (history 0, out_len 0).  The rows written may overlap neither the history
+ * read nor each other (nothing orders the copies).  Needs 16-byte aligned pointers and strides in whole
+ * 16-byte pieces, head_dim a multiple of 16 (bf16) or 8 (fp32), and no folded norm. */
 typedef struct {
   const void* k_hist; int64_t k_hist_stride_b, k_hist_stride_h, k_hist_stride_t; /* first of the last `history` rows */
   const void* v_hist; int64_t v_hist_stride_b, v_hist_stride_h, v_hist_stride_t;

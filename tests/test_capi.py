@@ -2,6 +2,7 @@
 ctypes structures match the C layout (checked against gcc's offsetof on the header).
 No kernel is launched: only host-side calls that return before touching a GPU."""
 import ctypes as C
+import hashlib
 import os
 import re
 import subprocess
@@ -36,6 +37,23 @@ def test_every_declared_symbol_is_exported_and_typed(lib):
         assert name in N.SIGNATURES, f"{name} has no ctypes signature"
         assert hasattr(lib, name), f"{name} not exported"
     assert set(N.SIGNATURES) == set(names)
+
+
+def test_declarations_belong_to_the_abi_version():
+    """Another set of structures, entry points or constants takes another UTTT_ABI_VERSION: a change to the
+    header's declarations changes the digest here, together with the version."""
+    text = re.sub(r"/\*.*?\*/", " ", open(HEADER).read(), flags=re.S)
+    text = " ".join(re.sub(r"#define UTTT_ABI_VERSION \d+", "", text).split())
+    assert (N.ABI_VERSION, hashlib.sha256(text.encode()).hexdigest()[:16]) == (25, "2b51cad2d8aee2fe")
+
+
+def test_library_of_another_version_is_refused(tmp_path, monkeypatch):
+    """Also where it lacks entry points of this one."""
+    (tmp_path / "old.c").write_text(f"int uttt_abi_version(void) {{ return {N.ABI_VERSION - 1}; }}\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(tmp_path / "old.so"), str(tmp_path / "old.c")], check=True)
+    monkeypatch.setattr(N, "_lib", None)
+    with pytest.raises(RuntimeError, match=f"ABI version {N.ABI_VERSION - 1}, expected {N.ABI_VERSION}"):
+        N.load_library(str(tmp_path / "old.so"))
 
 
 def test_struct_layouts_match_the_c_header(tmp_path):

@@ -292,13 +292,13 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
                 f"{path} is missing: the uTTT HIP kernels are not built "
                 "(run `python -m utttcompanion_amd.build`); there is no fallback path")
         lib = C.CDLL(path)
+        version = lib.uttt_abi_version()  # before the symbols: another version may lack some
+        if version != ABI_VERSION:
+            raise RuntimeError(f"{path} has ABI version {version}, expected {ABI_VERSION}: rebuild it")
         for name, (res, argt) in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = argt
-        version = lib.uttt_abi_version()
-        if version != ABI_VERSION:
-            raise RuntimeError(f"{path} has ABI version {version}, expected {ABI_VERSION}: rebuild it")
         _lib = lib
         return lib
 

@@ -1078,7 +1078,8 @@ def rope_kv_append(q: Tensor, k: Tensor, v: Tensor, cos: Tensor, sin: Tensor, st
 
     ``history`` = (k, v), (B | 1, Hkv, n, hd) each, goes to the caches' rows just before ``kv_offset``;
     ``out`` = (k, v), (B, Hkv, m, hd) with shared strides, receives the last m rows of history and new
-    ones together: in the same launch where the operands are 16-byte aligned, by copies otherwise."""
+    ones together: in the same launch where the operands are 16-byte aligned, by copies otherwise.  None
+    of the rows written may overlap another, or the history."""
     bsz, tokens, heads, hd = q.shape
     hkv = k.shape[2]
     if k.shape != (bsz, tokens, hkv, hd) or v.shape != k.shape:
