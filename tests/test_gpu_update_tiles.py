@@ -19,6 +19,12 @@ CASES = [
     (1, 300, 256, 192, "own", True, 0.01),    # five
     (8, 37, 320, 256, "shared", True, 1.0),
     (2, 40, 64, 8256, "own", True, 0.01),     # 129 norm partials, one past the straight loads
+    # the larger tiles, by the plan's rule (H's, Z's); K and Q rows of one matrix meet inside a tile
+    (16, 190, 512, 1024, "own", True, 1.0),   # 256 x 256, 64 x 128; three token blocks
+    (16, 300, 512, 1024, "own", False, 0.01), # 256 x 256, 128 x 128; five
+    (36, 300, 320, 256, "own", True, 1.0),    # 256 x 256 both; ragged columns
+    (36, 300, 320, 256, "other", False, 1.0), # 128 x 128 both, a matrix each
+    (26, 300, 512, 256, "shared", False, 1.0),# 256 x 256 both, a matrix each
 ]
 
 
@@ -70,9 +76,15 @@ def test_update_matches_float64(case, out):
         assert float((got - step).norm()) <= 2.0 ** -7 * float(step.norm()) + floor, ("s", i)
         new_w = torch.where(live.bool(), decay * w[i].double() + res[4 + i].double().cpu(), w[i].double())
         assert float((res[1 + i].double().cpu() - new_w).abs().max()) <= 4 * 2.0 ** -24 * float(new_w.abs().max()), ("w", i)
-    # the readout as in the frozen one: output rounding, and H's through the LayerNorm
-    bound = 2.0 ** -8 * ref[0].abs() + 7 * 2.0 ** -9 / 3 ** 0.5 * 2.0
-    assert bool(((res[0].double().cpu() - ref[0]).abs() <= bound).all())
+    # the readout as in the frozen one: the LayerNorm pair enters in the activation type; output rounding, and
+    # H's through the LayerNorm (with the pair in 64 bits, its own rounding, up to 2^-8 of LN(z) and of the bias,
+    # used the bound up at one of the 1.6 million elements of 16 x 190 x 512)
+    r = rd64 or w16
+    z = (torch.nn.functional.silu(q.double() @ r[1]) * (q.double() @ r[0])) @ r[2]
+    out64 = q.double() + torch.nn.functional.layer_norm(z, (d,), *(t.bfloat16().double() for t in ln), 1e-5)
+    assert float((out64 - ref[0]).abs().max()) <= 2.0 ** -8 * float((out64 - q.double()).abs().max() + ln[1].abs().max())
+    bound = 2.0 ** -8 * out64.abs() + 7 * 2.0 ** -9 / 3 ** 0.5 * 2.0
+    assert bool(((res[0].double().cpu() - out64).abs() <= bound).all())
     assert abs(float(res[7]) - float(ref[7])) <= 2.0 ** -8 * abs(float(ref[7]))
 
 
@@ -109,3 +121,64 @@ def test_clip_factor_of_similar_tokens(tokens, noise):
     # squares added up in fp32 in chains of at most 12 D / 64 + 20 additions, 2^-24 each; half of it in the
     # root, whose own rounding and the division's are 2^-23
     assert float((factor / want - 1).abs().max()) <= (12 * d / 64 + 20) * 2.0 ** -25 + 2.0 ** -22
+
+
+def gate_inputs(tokens, masked):
+    """Four rows with losses far apart: (chunk_update's first 14 arguments on the GPU, token counts)."""
+    b, d, f = 4, 128, 192
+    g = torch.Generator().manual_seed(tokens + masked)
+    unit = lambda: torch.nn.functional.rms_norm(torch.randn(b, tokens, d, generator=g), (d,))
+    q, k, v = unit(), unit(), unit() * torch.tensor([0.3, 1.0, 3.0, 10.0]).view(b, 1, 1)
+    eta, alpha = (x * torch.rand(b, tokens, 1, generator=g) for x in (0.015, 0.005))
+    w = [torch.randn(b, d, f, generator=g) / d ** 0.5, torch.randn(b, d, f, generator=g) / d ** 0.5,
+         torch.randn(b, f, d, generator=g) * 0.1 / f ** 0.5]
+    s = [1e-3 * torch.randn(t.shape, generator=g) for t in w]
+    ln = [1 + 0.1 * torch.randn(d, generator=g), 0.1 * torch.randn(d, generator=g)]
+    mask = None
+    if masked:
+        mask = torch.ones(b, tokens)
+        mask[1, tokens // 2:] = 0
+        mask[3, ::3] = 0
+    args = [t.bfloat16().cuda() for t in (q, k, v, eta, alpha)] + [t.cuda() for t in w + s + ln]
+    return args + [None if mask is None else mask.cuda()], mask.sum(1) if masked else torch.full((b,), float(tokens))
+
+
+@pytest.mark.parametrize("tokens", [37, 64, 129])  # the row scalars formed in the write, and in a launch of their own
+@pytest.mark.parametrize("masked", [False, True])
+def test_row_loss_and_inclusive_gate(tokens, masked):
+    """The per-row [sum of masked token losses, valid tokens] against float64, and the gate at a row's own
+    mean exactly: that row is written there and keeps W and S one float step above."""
+    import numpy as np
+    from utttcompanion_amd import kernels as K
+    args, counts = gate_inputs(tokens, masked)
+    print(f"row loss and gate {tokens} tokens, masked {masked}", flush=True)
+
+    def run(gate):
+        row_loss = torch.full((4, 2), float("nan"), device="cuda")
+        out = K.prepare_chunk_update(*args, 0.9, 1.0, True, 1e-5, row_loss=row_loss, min_row_surprise=gate).launch()
+        return [t.clone() for t in out], row_loss.cpu()
+
+    plain, rl = run(0.0)
+    assert torch.equal(rl[:, 1], counts)
+    means = rl[:, 0] / torch.clamp(rl[:, 1], min=1.0)  # as the kernels form it
+    k, v, w = args[1], args[2], args[5:8]
+    mask = args[13]
+    rows = om.row_surprise(k.double(), v.double(), *(t.bfloat16().double() for t in w), *(t.double() for t in args[11:13]),
+                           None if mask is None else mask.double(), True, 1e-5).cpu()
+    # H is rounded to bf16 (2^-8 relative at most), so LN(z), of unit size, is off by that a token at most, and a
+    # token's loss, half the mean square of an error e, by 2^-8 sqrt(2 loss) (and its square)
+    assert bool(((means.double() - rows).abs() <= 2.0 ** -8 * (2 * rows).sqrt() + 2.0 ** -16).all())
+    assert all(means[i] < means[i + 1] for i in range(3))
+    surprise = float(rl[:, 0].double().sum() / rl[:, 1].double().sum())
+    assert abs(float(plain[7]) - surprise) <= 1e-6 * surprise
+    start = args[5:11]
+    for r in range(4):
+        at = float(means[r])
+        for gate in (at, float(np.nextafter(np.float32(at), np.float32(np.inf)))):
+            got, rl2 = run(gate)
+            assert torch.equal(rl2, rl) and torch.equal(got[0], plain[0]) and torch.equal(got[7], plain[7])
+            for i in range(4):
+                kept = i < r or (i == r and gate > at)
+                for a, p, o in zip(got[1:7], plain[1:7], start):
+                    assert torch.equal(a[i], o[i] if kept else p[i]), (r, gate, i)
+    assert not any(torch.equal(p[i], o[i]) for p, o in zip(plain[1:7], start) for i in range(4))
