@@ -544,43 +544,42 @@ struct BwdArgs {
   const void* dz;  // (B, tok_pad, D)
   void* du;        // (B, tok_pad, F)
   void* dg;
-  float* nrm;      // (B, F/64), one token block only (longer chunks: k_apply<.., true>)
+  float* nrm;      // (B, F/64), one token block only (longer chunks: k_apply<true>)
 };
 
-template <typename T>
 __global__ void __launch_bounds__(kThreads) k_backward(const BwdArgs a) {
-  constexpr int LD = lds_ld<T>();
-  __shared__ __align__(16) T buf0[64 * LD];  // dZ rows, then K^T tiles
-  __shared__ __align__(16) T buf1[64 * LD];  // W_down rows, then dZ^T tiles
-  __shared__ __align__(16) T hts[64 * LD];   // H^T  [f][t]
-  __shared__ __align__(16) T dus[64 * LD];   // dU^T [f][t]
-  __shared__ __align__(16) T dgs[64 * LD];   // dG^T [f][t]
+  constexpr int LD = lds_ld<float>();
+  __shared__ __align__(16) float buf0[64 * LD];  // dZ rows, then K^T tiles
+  __shared__ __align__(16) float buf1[64 * LD];  // W_down rows, then dZ^T tiles
+  __shared__ __align__(16) float hts[64 * LD];   // H^T  [f][t]
+  __shared__ __align__(16) float dus[64 * LD];   // dU^T [f][t]
+  __shared__ __align__(16) float dgs[64 * LD];   // dG^T [f][t]
   __shared__ float red[4];
   const int ft = blockIdx.x, b = blockIdx.y, t0 = blockIdx.z * 64;  // token block blockIdx.z
   const int f0 = ft * 64;
   const int w = threadIdx.x >> 6, wr = (w >> 1) * 32, wc = (w & 1) * 32;
-  const T* dz = static_cast<const T*>(a.dz) + ((int64_t)b * a.tok_pad + t0) * a.D;
+  const float* dz = static_cast<const float*>(a.dz) + ((int64_t)b * a.tok_pad + t0) * a.D;
   const float* wd = a.wd + (int64_t)b * a.w_rs + (int64_t)f0 * a.D;
-  const T* kr = static_cast<const T*>(a.k) + (int64_t)b * a.k_rs;
+  const float* kr = static_cast<const float*>(a.k) + (int64_t)b * a.k_rs;
   const int64_t rowbase = ((int64_t)b * a.tok_pad + t0) * a.F + f0;
 
   // dH tile [t][f] over the full D (A = dZ rows, B^T = W_down rows)
   {
-    RowStage<T, KT> zst;
+    RowStage<float, KT> zst;
     RowStage<float, KT> wst;
     zst.load(dz, a.D, 64);
     wst.load(wd, a.D, 64);
     f32x16 acc;
     zero(acc);
     for (int d0 = 0; d0 < a.D; d0 += KT) {
-      zst.template store<T>(buf0, LD);
-      wst.template store<T>(buf1, LD);
+      zst.template store<float>(buf0, LD);
+      wst.template store<float>(buf1, LD);
       __syncthreads();
       if (d0 + KT < a.D) {
         zst.load(dz + d0 + KT, a.D, 64);
         wst.load(wd + d0 + KT, a.D, 64);
       }
-      wave_mma<T, KT>(acc, buf0 + wr * LD, LD, buf1 + wc * LD, LD);
+      wave_mma<float, KT>(acc, buf0 + wr * LD, LD, buf1 + wc * LD, LD);
       __syncthreads();
     }
     const int f = wc + acc_col();
@@ -591,46 +590,46 @@ __global__ void __launch_bounds__(kThreads) k_backward(const BwdArgs a) {
       const float u = a.u_store[off], g = a.g_store[off];
       const float sg = sigmoidf_acc(g);
       const float dh = acc[i];
-      const T du = from_f32<T>(dh * (g * sg));
-      const T dg = from_f32<T>(dh * u * (sg * (1.0f + g * (1.0f - sg))));
-      static_cast<T*>(a.du)[off] = du;
-      static_cast<T*>(a.dg)[off] = dg;
+      const float du = dh * (g * sg);
+      const float dg = dh * u * (sg * (1.0f + g * (1.0f - sg)));
+      static_cast<float*>(a.du)[off] = du;
+      static_cast<float*>(a.dg)[off] = dg;
       dus[f * LD + t] = du;
       dgs[f * LD + t] = dg;
     }
   }
   // with several token blocks the gradient norm needs every block's products: a later launch
-  // (k_apply<T, true>) forms it from the whole chunk
+  // (k_apply<true>) forms it from the whole chunk
   if (a.ntb > 1) return;
   // H^T for this F tile
   {
-    ColStage<T, 64> hst;
-    hst.load(static_cast<const T*>(a.h) + rowbase, a.F, 64, threadIdx.x);
-    hst.template store<T>(hts, LD);
+    ColStage<float, 64> hst;
+    hst.load(static_cast<const float*>(a.h) + rowbase, a.F, 64, threadIdx.x);
+    hst.template store<float>(hts, LD);
   }
 
   // |gW_up[:, tile]|^2 + |gW_gate[:, tile]|^2 (rows d) and |gW_down[tile, :]|^2 (cols d)
-  constexpr int kUnits = ColStage<T, 64>::kUnits;  // 64 (bf16) or 128 (fp32)
+  constexpr int kUnits = ColStage<float, 64>::kUnits;  // 128: both tiles at once
   const bool k_part = threadIdx.x < kUnits;
   const int unit = k_part ? threadIdx.x : threadIdx.x - kUnits;
-  ColStage<T, 64> cst;
-  const T* csrc = k_part ? kr : dz;
+  ColStage<float, 64> cst;
+  const float* csrc = k_part ? kr : dz;
   const int cvalid = k_part ? a.C : 64;
-  T* cdst = k_part ? buf0 : buf1;
+  float* cdst = k_part ? buf0 : buf1;
   cst.load(csrc, a.D, cvalid, unit < kUnits ? unit : kUnits);
   float sq = 0.f;
   for (int d0 = 0; d0 < a.D; d0 += 64) {
     __syncthreads();
-    cst.template store<T>(cdst, LD);
+    cst.template store<float>(cdst, LD);
     __syncthreads();
     if (d0 + 64 < a.D) cst.load(csrc + d0 + 64, a.D, cvalid, unit < kUnits ? unit : kUnits);
     f32x16 au, ag, ad;
     zero(au);
     zero(ag);
     zero(ad);
-    wave_mma<T, 64>(au, buf0 + wr * LD, LD, dus + wc * LD, LD);
-    wave_mma<T, 64>(ag, buf0 + wr * LD, LD, dgs + wc * LD, LD);
-    wave_mma<T, 64>(ad, hts + wr * LD, LD, buf1 + wc * LD, LD);
+    wave_mma<float, 64>(au, buf0 + wr * LD, LD, dus + wc * LD, LD);
+    wave_mma<float, 64>(ag, buf0 + wr * LD, LD, dgs + wc * LD, LD);
+    wave_mma<float, 64>(ad, hts + wr * LD, LD, buf1 + wc * LD, LD);
 #pragma unroll
     for (int i = 0; i < 16; ++i) sq += au[i] * au[i] + ag[i] * ag[i] + ad[i] * ad[i];
   }
@@ -666,7 +665,6 @@ struct ApplyArgs {
 
 // fp32 path: the last wave of an apply workgroup derives its row's clip factor, decay and active flag (and,
 // in the first workgroups, the row's loss sums and the batch-global surprise).
-template <typename T>
 __device__ __forceinline__ void apply_row_scalars(const ApplyArgs& a, int b, float* row_scalar) {
   {
     const int lane = threadIdx.x - 192;
@@ -674,7 +672,7 @@ __device__ __forceinline__ void apply_row_scalars(const ApplyArgs& a, int b, flo
     for (int i = lane; i < a.n_norm; i += 64) n2 += a.nrm[(int64_t)b * a.n_norm + i];
     n2 = wave_sum(n2);
     float asum = 0.f, msum = 0.f, any = 0.f;
-    const T* al = static_cast<const T*>(a.alpha) + (int64_t)b * a.alpha_rs;
+    const float* al = static_cast<const float*>(a.alpha) + (int64_t)b * a.alpha_rs;
     for (int t = lane; t < a.C; t += 64) {
       if (a.mask != nullptr) {
         const float mt = a.mask[(int64_t)b * a.mask_rs + t];
@@ -730,14 +728,13 @@ __device__ __forceinline__ void apply_row_scalars(const ApplyArgs& a, int b, flo
 // The same scalars once per row (bf16, several token blocks): out (B, 4) = clip factor, decay, active
 // flag.  Such a chunk has a norm partial per gradient tile (2112 at d 1024, F 2816), too many
 // for every workgroup of the apply to sum: that took most of its 147 us at 2 rows of 128 tokens.
-template <typename T>
 __global__ void __launch_bounds__(kThreads) k_row_scalars(const ApplyArgs a, float* out) {
   __shared__ float red[20];
   const int b = blockIdx.x;
   float v[5] = {0.f, 0.f, 0.f, 0.f, 0.f};  // squared norm, alpha sum, valid tokens, any valid, loss sum
   if (a.max_norm > 0.f)
     for (int i = threadIdx.x; i < a.n_norm; i += kThreads) v[0] += a.nrm[(int64_t)b * a.n_norm + i];
-  const T* al = static_cast<const T*>(a.alpha) + (int64_t)b * a.alpha_rs;
+  const bf16* al = static_cast<const bf16*>(a.alpha) + (int64_t)b * a.alpha_rs;
   for (int t = threadIdx.x; t < a.C; t += kThreads) {
     const float mt = a.mask != nullptr ? a.mask[(int64_t)b * a.mask_rs + t] : 1.f;
     v[1] += a.mask != nullptr ? to_f32(al[t]) * mt : to_f32(al[t]);
@@ -771,11 +768,11 @@ __global__ void __launch_bounds__(kThreads) k_row_scalars(const ApplyArgs a, flo
 
 // NORM: instead of applying, write the tile's squared Frobenius norm to nrm (one partial per tile):
 // the clip norm of a chunk longer than one token block, whose gradient tiles sum over its blocks.
-template <typename T, bool NORM = false>
+template <bool NORM>
 __global__ void __launch_bounds__(kThreads) k_apply(const ApplyArgs a) {
-  constexpr int LD = lds_ld<T>();
-  __shared__ __align__(16) T as[64 * LD];
-  __shared__ __align__(16) T bs[64 * LD];
+  constexpr int LD = lds_ld<float>();
+  __shared__ __align__(16) float as[64 * LD];
+  __shared__ __align__(16) float bs[64 * LD];
   __shared__ float row_scalar[3];
   __shared__ float red[4];
   const int nD = a.D / 64, nF = a.F / 64;
@@ -784,7 +781,7 @@ __global__ void __launch_bounds__(kThreads) k_apply(const ApplyArgs a) {
   const int w = threadIdx.x >> 6, wr = (w >> 1) * 32, wc = (w & 1) * 32;
 
   int r0, c0, ld_out;
-  const T *asrc, *bsrc;
+  const float *asrc, *bsrc;
   int64_t a_ld, b_ld;
   int a_valid;
   if (m < 2) {  // W_up / W_gate tile (d, f) = K^T dU / K^T dG
@@ -792,20 +789,20 @@ __global__ void __launch_bounds__(kThreads) k_apply(const ApplyArgs a) {
     r0 = dt * 64;
     c0 = ft * 64;
     ld_out = a.F;
-    asrc = static_cast<const T*>(a.k) + (int64_t)b * a.k_rs + r0;
+    asrc = static_cast<const float*>(a.k) + (int64_t)b * a.k_rs + r0;
     a_ld = a.D;
     a_valid = a.C;
-    bsrc = static_cast<const T*>(m == 0 ? a.du : a.dg) + (int64_t)b * a.tok_pad * a.F + c0;
+    bsrc = static_cast<const float*>(m == 0 ? a.du : a.dg) + (int64_t)b * a.tok_pad * a.F + c0;
     b_ld = a.F;
   } else {      // W_down tile (f, d) = H^T dZ
     const int ft = j / nD, dt = j - ft * nD;
     r0 = ft * 64;
     c0 = dt * 64;
     ld_out = a.D;
-    asrc = static_cast<const T*>(a.h) + (int64_t)b * a.tok_pad * a.F + r0;
+    asrc = static_cast<const float*>(a.h) + (int64_t)b * a.tok_pad * a.F + r0;
     a_ld = a.F;
     a_valid = a.tok_pad;  // rows past the chunk are zero
-    bsrc = static_cast<const T*>(a.dz) + (int64_t)b * a.tok_pad * a.D + c0;
+    bsrc = static_cast<const float*>(a.dz) + (int64_t)b * a.tok_pad * a.D + c0;
     b_ld = a.D;
   }
   // the state tile is the bulk of the traffic: issue its loads first
@@ -822,7 +819,7 @@ __global__ void __launch_bounds__(kThreads) k_apply(const ApplyArgs a) {
       sv[i] = ssrc[off];
     }
   }
-  constexpr int kUnits = ColStage<T, 64>::kUnits;
+  constexpr int kUnits = ColStage<float, 64>::kUnits;
   f32x16 acc;
   zero(acc);
   // the gradient tile: K = the chunk's tokens, one block of 64 per step
@@ -830,16 +827,16 @@ __global__ void __launch_bounds__(kThreads) k_apply(const ApplyArgs a) {
     const int t0 = tb * 64;
     if (tb > 0) __syncthreads();  // the previous block's products are done with as / bs
     {
-      ColStage<T, 64> cst;
+      ColStage<float, 64> cst;
       const bool a_part = threadIdx.x < kUnits;
       const int unit = a_part ? threadIdx.x : threadIdx.x - kUnits;
       cst.load(a_part ? asrc + (int64_t)t0 * a_ld : bsrc + (int64_t)t0 * b_ld, a_part ? a_ld : b_ld,
                a_part ? min(64, a_valid - t0) : 64, unit < kUnits ? unit : kUnits);
-      cst.template store<T>(a_part ? as : bs, LD);
+      cst.template store<float>(a_part ? as : bs, LD);
     }
-    if (!NORM && tb == 0 && threadIdx.x >= 192) apply_row_scalars<T>(a, b, row_scalar);
+    if (!NORM && tb == 0 && threadIdx.x >= 192) apply_row_scalars(a, b, row_scalar);
     __syncthreads();
-    wave_mma<T, 64>(acc, as + wr * LD, LD, bs + wc * LD, LD);
+    wave_mma<float, 64>(acc, as + wr * LD, LD, bs + wc * LD, LD);
   }
   if constexpr (NORM) {
     float sq = 0.f;
@@ -1013,16 +1010,16 @@ static void launch_update(const uttt_chunk_update_args& a, char* ws, const Updat
       if (ntb > 1 && a.max_inner_grad_norm > 0.f) launch_update_norm(u, st);
     }
     if (want(4)) {
-      if (ntb > 1) hipLaunchKernelGGL(k_row_scalars<T>, dim3(B), blk, 0, st, ap, scalars);
+      if (ntb > 1) hipLaunchKernelGGL(k_row_scalars, dim3(B), blk, 0, st, ap, scalars);
       launch_update_write(u, st);
     }
   } else {
     const dim3 tiles(3 * (D / 64) * (F / 64), B);
     if (want(3)) {
-      hipLaunchKernelGGL(k_backward<T>, dim3(F / 64, B, ntb), blk, 0, st, bw);
-      if (ntb > 1) hipLaunchKernelGGL((k_apply<T, true>), tiles, blk, 0, st, ap);
+      hipLaunchKernelGGL(k_backward, dim3(F / 64, B, ntb), blk, 0, st, bw);
+      if (ntb > 1) hipLaunchKernelGGL(k_apply<true>, tiles, blk, 0, st, ap);
     }
-    if (want(4)) hipLaunchKernelGGL((k_apply<T, false>), tiles, blk, 0, st, ap);
+    if (want(4)) hipLaunchKernelGGL(k_apply<false>, tiles, blk, 0, st, ap);
   }
 }
 

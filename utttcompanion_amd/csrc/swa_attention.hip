@@ -17,38 +17,19 @@
 namespace uttt {
 
 // ---------------------------------------------------------------------------
-// 16x16 MFMA wave tiles (used by attention)
-//   fp32: v_mfma_f32_16x16x4f32      (K = 4, lane supplies A[l%16][k0 + l/16])
-//   bf16: v_mfma_f32_16x16x32_bf16   (K = 32, lane supplies A[l%16][k0 + 8*(l/16) + 0..7])
-//   result: acc[i] = C[4*(l/16) + i][l%16]
+// 16x16 MFMA wave tiles (fp32 prefill attention): v_mfma_f32_16x16x4f32 (K = 4, lane supplies
+// A[l%16][k0 + l/16]), result acc[i] = C[4*(l/16) + i][l%16]
 // ---------------------------------------------------------------------------
-template <typename T> struct Mma16;
-template <> struct Mma16<float> {
-  static constexpr int kK = 4;
-  static constexpr int kPad = 4;  // rows stay 16-byte aligned
-  __device__ __forceinline__ static void step(f32x4& acc, const float* a_row, const float* b_row, int k0, int g) {
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a_row[k0 + g], b_row[k0 + g], acc, 0, 0, 0);
-  }
-};
-template <> struct Mma16<bf16> {
-  static constexpr int kK = 32;
-  static constexpr int kPad = 8;
-  __device__ __forceinline__ static void step(f32x4& acc, const bf16* a_row, const bf16* b_row, int k0, int g) {
-    const bf16x8 a = *reinterpret_cast<const bf16x8*>(a_row + k0 + 8 * g);
-    const bf16x8 b = *reinterpret_cast<const bf16x8*>(b_row + k0 + 8 * g);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-  }
-};
-
 // acc(16x16) += A(16 x KTOT) B(KTOT x 16); A rows at `a` ([16][lda]), B^T rows at `b` ([16][ldb])
-template <typename T, int KTOT>
-__device__ __forceinline__ void wave_mma16(f32x4& acc, const T* a, int lda, const T* b, int ldb) {
+template <int KTOT>
+__device__ __forceinline__ void wave_mma16(f32x4& acc, const float* a, int lda, const float* b, int ldb) {
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
-  const T* a_row = a + r * lda;
-  const T* b_row = b + r * ldb;
+  const float* a_row = a + r * lda;
+  const float* b_row = b + r * ldb;
 #pragma unroll
-  for (int k0 = 0; k0 < KTOT; k0 += Mma16<T>::kK) Mma16<T>::step(acc, a_row, b_row, k0, g);
+  for (int k0 = 0; k0 < KTOT; k0 += 4)
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a_row[k0 + g], b_row[k0 + g], acc, 0, 0, 0);
 }
 
 // RoPE for one element pair, rounding like the reference's activation-dtype ops:
@@ -213,16 +194,16 @@ __global__ void __launch_bounds__(kThreads) k_rope_roll(const uttt_rope_append_a
 }
 
 // ---------------------------------------------------------------------------
-// Prefill.  grid (q tiles of 64, n_heads, batch * nsplit): the key tiles that intersect a
+// Prefill, fp32.  grid (q tiles of 64, n_heads, batch * nsplit): the key tiles that intersect a
 // q tile's window are divided among `nsplit` workgroups; each wave owns 16 queries.  With
 // nsplit > 1 the workgroups write fp32 partials (row max, row sum, unnormalised output)
 // and k_swa_prefill_combine merges them.  Q / K rows are staged with 16-byte loads, V is
 // transposed in registers to [e][key]; the next key tile is loaded while the current one
 // is consumed.
 // ---------------------------------------------------------------------------
-template <typename T, int HD>
+template <int HD>
 struct AttnStage {
-  static constexpr int kVec = 16 / (int)sizeof(T);
+  static constexpr int kVec = 4;
   static constexpr int kChunksPerRow = HD / kVec;
   static constexpr int kRowChunks = 64 * kChunksPerRow / kThreads;  // per thread, for a 64-row tile
   static constexpr int kVUnits = 8 * kChunksPerRow;                 // 8 keys x one chunk per unit
@@ -232,15 +213,15 @@ struct AttnStage {
   // Branch-free: rows at or past n lie outside the buffer ranges and read as zeros, so the loads
   // carry no condition and the compiler has no reason to wait for them before the current tile's
   // work (a conditional load made it wait for every outstanding load right away).
-  __device__ __forceinline__ void load(const T* k, const T* v, int64_t st_k, int64_t st_v, int n) {
-    const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(k, (uint32_t)(max(n, 0) * st_k * (int64_t)sizeof(T)));
-    const __amdgpu_buffer_rsrc_t rv = buffer_rsrc(v, (uint32_t)(max(n, 0) * st_v * (int64_t)sizeof(T)));
+  __device__ __forceinline__ void load(const float* k, const float* v, int64_t st_k, int64_t st_v, int n) {
+    const __amdgpu_buffer_rsrc_t rk = buffer_rsrc(k, (uint32_t)(max(n, 0) * st_k * (int64_t)sizeof(float)));
+    const __amdgpu_buffer_rsrc_t rv = buffer_rsrc(v, (uint32_t)(max(n, 0) * st_v * (int64_t)sizeof(float)));
 #pragma unroll
     for (int j = 0; j < kRowChunks; ++j) {
       const int idx = threadIdx.x + j * kThreads;
       const int row = idx / kChunksPerRow, c = idx - row * kChunksPerRow;
       kr[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                            rk, (int)((row * st_k + c * kVec) * (int64_t)sizeof(T)), 0, 0));
+                                            rk, (int)((row * st_k + c * kVec) * (int64_t)sizeof(float)), 0, 0));
     }
     if (threadIdx.x < kVUnits) {
       const int kg = threadIdx.x / kChunksPerRow, c = threadIdx.x - kg * kChunksPerRow;
@@ -248,12 +229,12 @@ struct AttnStage {
       for (int i = 0; i < 8; ++i) {
         const int row = kg * 8 + i;
         vr[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                              rv, (int)((row * st_v + c * kVec) * (int64_t)sizeof(T)), 0, 0));
+                                              rv, (int)((row * st_v + c * kVec) * (int64_t)sizeof(float)), 0, 0));
       }
     }
   }
   template <int LQ, int LV>
-  __device__ __forceinline__ void store(T* ks, T* vt) const {
+  __device__ __forceinline__ void store(float* ks, float* vt) const {
 #pragma unroll
     for (int j = 0; j < kRowChunks; ++j) {
       const int idx = threadIdx.x + j * kThreads;
@@ -264,22 +245,15 @@ struct AttnStage {
       const int kg = threadIdx.x / kChunksPerRow, c = threadIdx.x - kg * kChunksPerRow;
 #pragma unroll
       for (int e = 0; e < kVec; ++e) {
-        T* d = vt + (c * kVec + e) * LV + kg * 8;
-        if constexpr (sizeof(T) == 2) {
-          bf16x8 o;
+        float* d = vt + (c * kVec + e) * LV + kg * 8;
+        f32x4 o0, o1;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) o[i] = from_f32<T>(Lanes16<bf16>::get(vr[i], e));
-          *reinterpret_cast<bf16x8*>(d) = o;
-        } else {
-          f32x4 o0, o1;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            o0[i] = Lanes16<float>::get(vr[i], e);
-            o1[i] = Lanes16<float>::get(vr[i + 4], e);
-          }
-          *reinterpret_cast<f32x4*>(d) = o0;
-          *reinterpret_cast<f32x4*>(d + 4) = o1;
+        for (int i = 0; i < 4; ++i) {
+          o0[i] = Lanes16<float>::get(vr[i], e);
+          o1[i] = Lanes16<float>::get(vr[i + 4], e);
         }
+        *reinterpret_cast<f32x4*>(d) = o0;
+        *reinterpret_cast<f32x4*>(d + 4) = o1;
       }
     }
   }
@@ -340,16 +314,16 @@ __device__ __forceinline__ float row16_sum(float v) {
 // fp32 and bf16 tolerances of the attention output
 __device__ __forceinline__ float exp_fast(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
 
-template <typename T, int HD>
+template <int HD>
 __global__ void __launch_bounds__(kThreads) k_swa_prefill(const uttt_swa_prefill_args a, float* part, int nsplit,
                                                           int tiles_per_split, int q_pad, int nqt) {
-  constexpr int PAD = Mma16<T>::kPad;
+  constexpr int PAD = 4;         // rows stay 16-byte aligned
   constexpr int LQ = HD + PAD;   // q/k rows [token][e]
   constexpr int LV = 64 + PAD;   // v^T rows [e][key], p rows [query][key]
-  __shared__ __align__(16) T qs[64 * LQ];
-  __shared__ __align__(16) T ks[64 * LQ];
-  __shared__ __align__(16) T vt[HD * LV];
-  __shared__ __align__(16) T ps[64 * LV];
+  __shared__ __align__(16) float qs[64 * LQ];
+  __shared__ __align__(16) float ks[64 * LQ];
+  __shared__ __align__(16) float vt[HD * LV];
+  __shared__ __align__(16) float ps[64 * LV];
   // the workgroups of one (row, kv head) read the same keys and values: they are placed as the
   // tiles of one row (row_tile), split fastest, then the query heads of the kv head, then q tiles
   const int rep = (int)(a.n_heads / a.n_kv_heads);
@@ -377,11 +351,11 @@ __global__ void __launch_bounds__(kThreads) k_swa_prefill(const uttt_swa_prefill
     return;
   }
 
-  const T* qg = static_cast<const T*>(a.q) + b * a.q_stride_b + h * a.q_stride_h;
-  const T* kg = static_cast<const T*>(a.k) + b * a.k_stride_b + kvh * a.k_stride_h;
-  const T* vg = static_cast<const T*>(a.v) + b * a.v_stride_b + kvh * a.v_stride_h;
+  const float* qg = static_cast<const float*>(a.q) + b * a.q_stride_b + h * a.q_stride_h;
+  const float* kg = static_cast<const float*>(a.k) + b * a.k_stride_b + kvh * a.k_stride_h;
+  const float* vg = static_cast<const float*>(a.v) + b * a.v_stride_b + kvh * a.v_stride_h;
   {
-    constexpr int kVec = 16 / (int)sizeof(T), kCpr = HD / kVec;
+    constexpr int kVec = 4, kCpr = HD / kVec;
     for (int idx = threadIdx.x; idx < 64 * kCpr; idx += kThreads) {
       const int r = idx / kCpr, cc = idx - r * kCpr;
       *reinterpret_cast<uint4*>(qs + r * LQ + cc * kVec) =
@@ -399,7 +373,7 @@ __global__ void __launch_bounds__(kThreads) k_swa_prefill(const uttt_swa_prefill
 #pragma unroll
   for (int t = 0; t < HD / 16; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  AttnStage<T, HD> stg;
+  AttnStage<HD> stg;
   {
     const int64_t kt0 = lo + (int64_t)t_begin * 64;
     stg.load(kg + kt0 * a.k_stride_t, vg + kt0 * a.v_stride_t, a.k_stride_t, a.v_stride_t,
@@ -421,7 +395,7 @@ __global__ void __launch_bounds__(kThreads) k_swa_prefill(const uttt_swa_prefill
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
       s[n] = f32x4{0.f, 0.f, 0.f, 0.f};
-      wave_mma16<T, HD>(s[n], qs + (16 * w) * LQ, LQ, ks + (16 * n) * LQ, LQ);
+      wave_mma16<HD>(s[n], qs + (16 * w) * LQ, LQ, ks + (16 * n) * LQ, LQ);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -452,22 +426,22 @@ __global__ void __launch_bounds__(kThreads) k_swa_prefill(const uttt_swa_prefill
 #pragma unroll
       for (int t = 0; t < HD / 16; ++t) o[t][i] *= corr;
 #pragma unroll
-      for (int n = 0; n < 4; ++n) ps[(16 * w + 4 * g + i) * LV + 16 * n + c] = from_f32<T>(s[n][i]);
+      for (int n = 0; n < 4; ++n) ps[(16 * w + 4 * g + i) * LV + 16 * n + c] = s[n][i];
     }
     __syncthreads();
 #pragma unroll
-    for (int t = 0; t < HD / 16; ++t) wave_mma16<T, 64>(o[t], ps + (16 * w) * LV, LV, vt + (16 * t) * LV, LV);
+    for (int t = 0; t < HD / 16; ++t) wave_mma16<64>(o[t], ps + (16 * w) * LV, LV, vt + (16 * t) * LV, LV);
   }
 
   if (nsplit == 1) {
-    T* og = static_cast<T*>(a.out) + b * a.o_stride_b + h * a.o_stride_h;
+    float* og = static_cast<float*>(a.out) + b * a.o_stride_b + h * a.o_stride_h;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int qi = q0 + 16 * w + 4 * g + i;
       if (qi >= a.q_len) continue;
       const float inv = l_run[i] > 0.f ? 1.0f / l_run[i] : 0.f;
 #pragma unroll
-      for (int t = 0; t < HD / 16; ++t) og[(int64_t)qi * a.o_stride_t + 16 * t + c] = from_f32<T>(o[t][i] * inv);
+      for (int t = 0; t < HD / 16; ++t) og[(int64_t)qi * a.o_stride_t + 16 * t + c] = o[t][i] * inv;
     }
   } else {
 #pragma unroll
@@ -1075,7 +1049,7 @@ static void launch_prefill(const uttt_swa_prefill_args& a, const PrefillPlan& p,
     launch_swa_prefill_mm(a, part, p.q_pad, st);
   } else {
     const dim3 grid((unsigned)row_tile_blocks((int)(a.batch * a.n_kv_heads), p.nqt * (int)(a.n_heads / a.n_kv_heads) * p.nsplit));
-    hipLaunchKernelGGL((k_swa_prefill<T, HD>), grid, dim3(kThreads), 0, st, a, part, p.nsplit, p.tiles_per_split,
+    hipLaunchKernelGGL(k_swa_prefill<HD>, grid, dim3(kThreads), 0, st, a, part, p.nsplit, p.tiles_per_split,
                        p.q_pad, p.nqt);
   }
   if (p.nsplit > 1)
