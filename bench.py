@@ -56,7 +56,7 @@ C3 = dict(vocab_size=32000, d_model=2048, n_layers=24, n_heads=16, n_kv_heads=4,
           sliding_window_size=1024, chunk_size=64, max_seq_len=4096)
 C3_BATCH, C3_SEQ = 4, 4096
 C5_REQUESTS, C5_LENGTHS = 16, (128, 4096)
-PHASES = ("k_up_gate", "k_down_partial", "k_ln_grad+k_ln_readout", "k_backward", "k_apply")
+PHASES = ("k_readout_mm (gated)", "k_readout_mm (down)", "k_ln_both", "k_update_back", "k_update_write")
 
 
 def measured_traffic(kernel: str, config: str = "c2"):
