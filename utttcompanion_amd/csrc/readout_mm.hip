@@ -18,8 +18,8 @@
 // with ranges the compiler could not prove uniform, each load became a loop over the distinct
 // descriptors of a wave (28 against 24 us at 1 x 333 tokens, d 768, F 2048).  Measured for the
 // whole readout against the 64 x 64-tile kernels it replaced: 4 x 2048 tokens, d 2048, F 5504, bf16
-// copies 1541 -> 557 us (995 TFLOP/s), fp32 masters 2510 -> 704 us; 2 x 333 tokens, d 768, F 2048
-// 39 -> 26 us and 35 -> 34 us; 128 tokens, d 2048, F 5504 53 -> 33 us and 62 -> 45 us.
+// copies 1536 -> 561 us (988 TFLOP/s), fp32 masters 2524 -> 683 us; 2 x 333 tokens, d 768, F 2048
+// 39 -> 28 us and 34 -> 33 us; 128 tokens, d 2048, F 5504 52 -> 33 us and 60 -> 44 us.
 #include "readout_mm.h"
 
 #include <algorithm>

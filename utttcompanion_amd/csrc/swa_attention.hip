@@ -101,8 +101,8 @@ __global__ void __launch_bounds__(kThreads) k_rope_append(const uttt_rope_append
 // rows copied in front of the appended ones, and the last out_len rows copied to a new cache.
 // Without a folded norm the pieces of all tokens and history rows of a row form one list, a piece
 // per thread (XN: a workgroup per token, whose threads first meet for the row's scale).  Bound by the
-// bytes: 4 x 4096 tokens, 16 + 2 x 4 heads of 128: 65 us a token row per workgroup in 2-byte
-// accesses, 45 us so, and the cache copies (11 us in two launches, 17 in four with history) gone.
+// bytes: 4 x 4096 tokens, 16 + 2 x 4 heads of 128: 63 us a token row per workgroup in 2-byte
+// accesses, 36 us so (6.1 TB/s), and the cache copies (11 us in two launches, 17 in four with history) gone.
 template <typename T> struct Piece16;
 template <> struct Piece16<bf16> { using type = bf16x8; };
 template <> struct Piece16<float> { using type = f32x4; };

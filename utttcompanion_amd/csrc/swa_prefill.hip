@@ -17,15 +17,17 @@
 //
 // The running maximum is raised whenever a tile's scores exceed it, so that a query's heaviest weight
 // is 1 exactly: the sum is formed from the unrounded weights, and a heaviest weight rounded to bf16
-// would be off from its share of it.  (Raising it only past a factor of 2^8 saved most of the output's
-// rescaling, and took the relative error at scores of standard deviation 4 from 1.7e-3 to 2.1e-3.)
+// would be off from its share of it.  (Raising it only past a factor of 2^8 saves most of the output's
+// rescaling, 167 instead of 174 us for the first call below, and takes the relative error at scores of
+// standard deviation 4 from 1.7e-3 to 2.1e-3.)
 //
 // What bounds it: LDS reads (each wave reads the whole K and V tile for its 32 queries, 32 KB per
 // 1024 MFMA cycles at head_dim 128) about equal to the MFMAs, with the softmax's vector work between
 // them.  Measured against the 16 x 16-tile kernel it replaced (64 queries per workgroup, V
 // transposed through registers): 4 x 4096 queries, 16 heads on 4, head_dim 128, window 1024:
-// 470 -> 183 us (645 TFLOP/s of visible pairs); 3 x 777 over 1288 keys, head_dim 64, window 512:
-// 28.9 -> 17.9 us; one 64-token chunk of 4 rows over 1088 keys, head_dim 128: 26.2 -> 21.5 us.
+// 485 -> 174 us (690 TFLOP/s of visible pairs); 3 x 777 over 1288 keys, head_dim 64, window 512:
+// 31.0 -> 19.4 us; one 64-token chunk of 4 rows over 1087 keys, head_dim 128, with the combine:
+// 25.7 -> 19.2 us.
 #include "swa_prefill.h"
 
 #include <math.h>
@@ -341,7 +343,8 @@ __global__ void __launch_bounds__(NW * 64, NW >= 6 ? 1 : 2) k_swa_prefill_mm(con
 constexpr int kMaxSplits = 16;
 
 // Key splits so that about kWantedWgs workgroups of four units exist.  Splitting costs partials and a
-// second launch (about 8 us), so it stops short of one workgroup per CU: 3 x 777 queries over 1288
+// second launch (about 8 us), so it stops short of one workgroup per CU (timed before the running maximum
+// was raised on every tile, which adds 4 to 8%): 3 x 777 queries over 1288
 // keys (12 heads on 4, window 512), 228 workgroups of three waves: 17.9 us unsplit, 28.5 us in two;
 // one 64-token chunk of 8 rows over 576 keys (64 workgroups): 13.7 us in three splits, 15.9 us in
 // four; 4 rows of 64 tokens over 1088 keys, head_dim 128 (32 workgroups): 21 us in four to eight.

@@ -8,10 +8,10 @@
 // The write is bound by the state it streams (48 D F bytes per row), the backward pass by the
 // latency of its D loop on few workgroups.  Measured against the register-staged kernels they
 // replaced (backward with the norm / state write with the row scalars, us):
-//   1 row x 37 tokens, d 768, F 2048      26 -> 14 / 23 -> 18
-//   8 rows x 64 tokens, d 768, F 2048     32 -> 17 / 163 -> 123 (604 MB, 4.9 TB/s)
-//   4 rows x 64 tokens, d 2048, F 5504    89 -> 40 / 569 -> 415 (5.2 TB/s)
-//   2 rows x 128 tokens, d 1024, F 2816   55 -> 26 / 146 -> 61
+//   1 row x 37 tokens, d 768, F 2048      28 -> 16 / 22 -> 14
+//   8 rows x 64 tokens, d 768, F 2048     30 -> 20 / 146 -> 106 (604 MB, 5.7 TB/s)
+//   4 rows x 64 tokens, d 2048, F 5504    91 -> 56 / 531 -> 398 (2.16 GB, 5.4 TB/s)
+//   2 rows x 128 tokens, d 1024, F 2816   54 -> 25 / 147 -> 56
 #include "update_mm.h"
 
 #include "uttt_device.h"
@@ -76,8 +76,8 @@ __device__ __forceinline__ void lds_write_b16(uint32_t addr, bf16 v) {
 // One (F tile, row, token block).  NORM (one token block): then the tile's squared gradient norm, the
 // sum of the squares of the gradient tiles K^T dU, K^T dG and dZ^T H, 64 x 64 each, in a second loop
 // over D whose first slabs arrive while dU and dG are formed.  (Gram matrices, <K K^T, dU dU^T> and
-// alike, need no second loop, but their terms have both signs: 1e-6 relative on independent tokens,
-// 1e-2 and more once a chunk's keys are nearly one token.)
+// alike, need no second loop and took 14, 17 and 40 us at the first three shapes above, but their terms
+// have both signs: 1e-6 relative on independent tokens, 1e-2 and more once a chunk's keys are nearly one.)
 template <bool NORM>
 __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArgs a) {
   constexpr int SLOT = 2 * 8192;      // dZ rows by direct loads, W_down rows rounded through registers
@@ -270,8 +270,8 @@ __global__ void __launch_bounds__(kThreads, 2) k_update_back(const UpdateBackArg
 //
 // kNormOnly: only the tile's squared norm.  kScalarsGiven: the row scalars are read.  kFormScalars
 // (one token block, F / 64 norm partials): every workgroup's first wave forms them while the slabs
-// and the state are on their way, instead of a launch of their own in front: a 37-token chunk at
-// d 768, F 2048 55.7 -> 53.8 us, a layer of 8 x 512 tokens (eight chunks) 1519 -> 1494 us.
+// and the state are on their way.  Against a launch of their own in front, that is 1.9 us less for a
+// 37-token chunk at d 768, F 2048 (of 55.7) and 25 us for eight chunks of 8 x 64 tokens (of 1519).
 enum WriteForm { kNormOnly, kScalarsGiven, kFormScalars };
 
 __device__ __forceinline__ float load_f32(const float* p, uint32_t bytes, int off) {
