@@ -16,6 +16,7 @@ SHAPES = [
     (4, 1025, 512, 1024),   # the wide tiles, one row past them
     (8, 700, 1024, 2816),   # the wide tiles, ragged rows
     (1, 2048, 2048, 5504),
+    (4, 250, 512, 1024),    # fp32 W: the down product in 64 x 64 tiles, at its smallest number of them
     (8, 100, 768, 2048),    # shared W: the rows' tiles next to each other
     (3, 129, 320, 8256),    # the same with ragged columns
 ]

@@ -1232,13 +1232,18 @@ struct ReadoutLayout {
   int nsplit, ntb;
 };
 
+// Splits of the down product of more than one token block, bf16 activations.
+static int long_down_splits(int64_t B, int64_t T, int64_t D, int64_t F, bool w_fp32) {
+  return readout_mm_down(B, T, D, F, w_fp32) ? readout_mm_splits(B, T, D, F, w_fp32)
+                                             : pick_nsplit((D / 64) * B * ((T + 63) / 64), F / 64);
+}
+
 static ReadoutLayout readout_layout(int64_t B, int64_t T, int64_t D, int64_t F, int32_t dtype) {
   ReadoutLayout L;
   L.ntb = (int)((T + 63) / 64);
-  // long bf16 blocks: the products of readout_mm.hip, whose split depends on the weights' type;
-  // the workspace holds either
+  // long bf16 blocks: the split depends on the weights' type; the workspace holds either
   L.nsplit = L.ntb > 1 && dtype == UTTT_DTYPE_BF16
-                 ? std::max(readout_mm_splits(B, T, D, F, false), readout_mm_splits(B, T, D, F, true))
+                 ? std::max(long_down_splits(B, T, D, F, false), long_down_splits(B, T, D, F, true))
                  : pick_nsplit((D / 64) * B * L.ntb, F / 64);
   // one token: room for the GEMV's F-block partials too
   const int64_t zsplits = T == 1 ? std::max<int64_t>(L.nsplit, F / gemv_fb(F)) : L.nsplit;
@@ -1300,10 +1305,14 @@ static void launch_readout(const uttt_readout_args& a, char* ws, const ReadoutLa
       m.w_up = a.w_up; m.w_gate = a.w_gate; m.w_down = a.w_down; m.w_rs = a.w_row_stride;
       m.w_fp32 = sizeof(WT) == 4;
       m.h = f.h[0]; m.zp = f.zp;
-      launch_readout_mm(m, st);
+      launch_readout_up(m, st);
+      f.nsplit = long_down_splits(B, a.tokens, D, F, m.w_fp32);
+      if (readout_mm_down(B, a.tokens, D, F, m.w_fp32))
+        launch_readout_down(m, st);
+      else if constexpr (sizeof(WT) == 4)
+        hipLaunchKernelGGL((k_down_partial<T, WT>), dim3(D / 64, f.nsplit, L.ntb * B), blk, 0, st, f);
       LnOutArgs o{};
-      o.B = B; o.ntok = (int)a.tokens; o.D = D; o.tok_pad = f.tok_pad; o.eps = a.eps;
-      o.nsplit = readout_mm_splits(B, a.tokens, D, F, m.w_fp32);
+      o.B = B; o.ntok = (int)a.tokens; o.D = D; o.tok_pad = f.tok_pad; o.eps = a.eps; o.nsplit = f.nsplit;
       o.zp = f.zp; o.x = a.x; o.x_rs = a.x_row_stride; o.ln_w = a.ln_weight; o.ln_b = a.ln_bias;
       o.out = a.out; o.out_rs = a.out_row_stride;
       launch_ln_readout<T>(dim3((unsigned)a.tokens, B), st, o);

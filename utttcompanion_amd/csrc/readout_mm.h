@@ -19,7 +19,7 @@ struct ReadoutMmArgs {
   int64_t w_rs;        // 0: shared
   bool w_fp32;
   void* h;     // bf16 (B, tok_pad, F)
-  float* zp;   // fp32 (readout_mm_splits(..), B, tok_pad, D)
+  float* zp;   // fp32 (splits, B, tok_pad, D)
 };
 
 // The forward products of a chunk update (K rows through the cursor weights, Q rows through the read
@@ -47,9 +47,11 @@ int update_mm_splits(int64_t B, int64_t T, int64_t D, int64_t F, bool joint, int
 void launch_update_up(const UpdateMmArgs& a, bool joint, hipStream_t st);
 void launch_update_down(const UpdateMmArgs& a, bool joint, hipStream_t st);
 
-// How many partials the down product leaves for the LayerNorm to sum.
+// The two products of the readout.  The down product leaves readout_mm_splits partials for the LayerNorm
+// to sum; where readout_mm_down is false, k_down_partial is the better one.
+bool readout_mm_down(int64_t B, int64_t T, int64_t D, int64_t F, bool w_fp32);
 int readout_mm_splits(int64_t B, int64_t T, int64_t D, int64_t F, bool w_fp32);
-
-void launch_readout_mm(const ReadoutMmArgs& a, hipStream_t st);
+void launch_readout_up(const ReadoutMmArgs& a, hipStream_t st);
+void launch_readout_down(const ReadoutMmArgs& a, hipStream_t st);
 
 }  // namespace uttt

@@ -361,7 +361,10 @@ int tile_cols(MmTile t) { return t == kWide ? 256 : 128; }
 // step's time of that shape, and a last partial round between a step's time at one workgroup per
 // CU and that.  The step times are the fit to readouts timed with every tile shape and split
 // forced, bf16 copies and fp32 masters, 100 to 16384 tokens at the model widths (d 512 to 2048);
-// the plan is then within 6% of the best forced one on each of them.  Wide tiles win where they
+// the plan is then within 6% of the best forced one on each of them.  Those of the gated product from
+// fp32 W are the fit to that product alone over 290 readouts of 1 to 8 rows of 65 to 1500 tokens (0.2%
+// from the best tile on average, 18% at most; with the down product's times 1.5% and 25%, and at 4 x 65
+// tokens, d 1024, F 2816 the small tile's 26.0 us instead of the middle one's 23.8).  Wide tiles win where they
 // fill the GPU, by reading each operand fewer times (4 x 2048 tokens, d 2048, F 5504, bf16: 950 /
 // 778 / 700 us with H in small / mid / wide tiles, then 701 / 622 / 557 us with Z in them); smaller
 // ones as soon as wide tiles leave CUs idle (2 x 333 tokens, d 768, F 2048: 32 / 35 / 48 us) or end
@@ -371,9 +374,11 @@ struct MmPlan {
   int splits;
 };
 
-MmPlan plan_mm(int64_t B, int64_t rows, int64_t cols, int64_t steps, int max_splits, bool w_fp32) {
-  constexpr double kFull[2][3] = {{0.87, 1.01, 1.89}, {1.40, 1.36, 2.30}};
-  constexpr double kLone[2][3] = {{0.42, 0.90, 1.82}, {0.60, 1.02, 1.50}};
+enum MmSteps { kBf16, kF32, kF32Readout };  // whose step times: kF32Readout the readout's gated product
+
+MmPlan plan_mm(int64_t B, int64_t rows, int64_t cols, int64_t steps, int max_splits, MmSteps of) {
+  constexpr double kFull[3][3] = {{0.87, 1.01, 1.89}, {1.40, 1.36, 2.30}, {1.40, 1.20, 2.10}};
+  constexpr double kLone[3][3] = {{0.42, 0.90, 1.82}, {0.60, 1.02, 1.50}, {0.70, 0.90, 2.00}};
   constexpr int kPlaces[3] = {512, 512, 256}, kCus = 256;
   const double z_us = (double)B * rows * cols * 8.0 / 4e6;  // one more set of partials, written and read
   MmPlan best{kSmall, 1};
@@ -384,10 +389,10 @@ MmPlan plan_mm(int64_t B, int64_t rows, int64_t cols, int64_t steps, int max_spl
       const int64_t n = B * ceil_div(rows, tile_rows(tile)) * ceil_div(cols, tile_cols(tile)) * s;
       const int64_t full = n / kPlaces[t], rest = n % kPlaces[t];
       const double k = (double)ceil_div(steps, s);
-      double us = full * (k * kFull[w_fp32][t] + 2.0) + (s - 1) * z_us;
+      double us = full * (k * kFull[of][t] + 2.0) + (s - 1) * z_us;
       if (rest > 0) {
         const double more = (double)std::max<int64_t>(0, rest - kCus) / kCus;
-        us += k * (kLone[w_fp32][t] + more * (kFull[w_fp32][t] - kLone[w_fp32][t])) + 2.0;
+        us += k * (kLone[of][t] + more * (kFull[of][t] - kLone[of][t])) + 2.0;
       }
       if (us < best_us) {
         best_us = us;
@@ -421,23 +426,8 @@ void launch_mm(MmArgs m, MmPlan p, hipStream_t st) {
 
 constexpr int kMaxSplits = 8;
 MmPlan plan_down(int64_t B, int64_t T, int64_t D, int64_t F, bool w_fp32) {
-  return plan_mm(B, ceil_div(T, 64) * 64, D, F / 64, (int)std::min<int64_t>(kMaxSplits, F / 64), w_fp32);
-}
-
-template <typename WT>
-void launch_both(const ReadoutMmArgs& a, hipStream_t st) {
-  MmArgs m{};
-  m.B = a.B; m.nseg = 1; m.rows = a.T; m.rows_pad = a.tok_pad; m.K = a.D; m.N = a.F;
-  m.a[0] = static_cast<const bf16*>(a.x); m.a_rs[0] = a.x_rs; m.a_ld = a.D;
-  m.w[0][0] = a.w_up; m.w[0][1] = a.w_gate; m.w_rs[0] = a.w_rs;
-  m.h[0] = static_cast<bf16*>(a.h);
-  launch_mm<true, WT>(m, plan_mm(a.B, a.tok_pad, 2 * (int64_t)a.F, a.D / 64, 1, a.w_fp32), st);
-  MmArgs z{};
-  z.B = a.B; z.nseg = 1; z.rows = a.tok_pad; z.rows_pad = a.tok_pad; z.K = a.F; z.N = a.D;
-  z.a[0] = static_cast<const bf16*>(a.h); z.a_rs[0] = (int64_t)a.tok_pad * a.F; z.a_ld = a.F;
-  z.w[0][0] = a.w_down; z.w_rs[0] = a.w_rs;
-  z.zp = a.zp;
-  launch_mm<false, WT>(z, plan_down(a.B, a.T, a.D, a.F, a.w_fp32), st);
+  return plan_mm(B, ceil_div(T, 64) * 64, D, F / 64, (int)std::min<int64_t>(kMaxSplits, F / 64),
+                 w_fp32 ? kF32 : kBf16);
 }
 
 }  // namespace
@@ -446,10 +436,18 @@ int readout_mm_splits(int64_t B, int64_t T, int64_t D, int64_t F, bool w_fp32) {
   return plan_down(B, T, D, F, w_fp32).splits;
 }
 
+// From fp32 W the small tile is slower than k_down_partial's 64 x 64 one from 128 of those on, when two of
+// them on a CU hide each other's loads: 3% with the LayerNorm over 122 readouts of 1 to 8 rows of 65 to
+// 1500 tokens at the model widths, up to 18% (2 x 700 tokens at d 512: 12.2 against 9.1 us).  Below that it
+// leaves fewer splits for the LayerNorm to sum: 4% faster over 94 of them.
+bool readout_mm_down(int64_t B, int64_t T, int64_t D, int64_t F, bool w_fp32) {
+  return !w_fp32 || B * ceil_div(T, 64) * (D / 64) < 128 || plan_down(B, T, D, F, true).tile != kSmall;
+}
+
 static MmPlan plan_update_down(int64_t B, int64_t T, int64_t D, int64_t F, bool joint, int most) {
   const int64_t rows = ceil_div(T, 64) * 64;
   return plan_mm(joint ? B : 2 * B, joint ? 2 * rows : rows, D, F / 64,
-                 (int)std::min<int64_t>(std::min(most, kMaxSplits), F / 64), true);
+                 (int)std::min<int64_t>(std::min(most, kMaxSplits), F / 64), kF32);
 }
 
 int update_mm_splits(int64_t B, int64_t T, int64_t D, int64_t F, bool joint, int most) {
@@ -467,7 +465,7 @@ void launch_update_up(const UpdateMmArgs& a, bool joint, hipStream_t st) {
   }
   m.u = a.u_store; m.g = a.g_store;
   launch_mm<true, float>(m, plan_mm(joint ? a.B : 2 * a.B, joint ? 2 * a.tok_pad : a.tok_pad, 2 * (int64_t)a.F,
-                                    a.D / 64, 1, true), st);
+                                    a.D / 64, 1, kF32), st);
 }
 
 void launch_update_down(const UpdateMmArgs& a, bool joint, hipStream_t st) {
@@ -482,11 +480,30 @@ void launch_update_down(const UpdateMmArgs& a, bool joint, hipStream_t st) {
   launch_mm<false, float>(z, plan_update_down(a.B, a.T, a.D, a.F, joint, a.splits), st);
 }
 
-void launch_readout_mm(const ReadoutMmArgs& a, hipStream_t st) {
+void launch_readout_up(const ReadoutMmArgs& a, hipStream_t st) {
+  MmArgs m{};
+  m.B = a.B; m.nseg = 1; m.rows = a.T; m.rows_pad = a.tok_pad; m.K = a.D; m.N = a.F;
+  m.a[0] = static_cast<const bf16*>(a.x); m.a_rs[0] = a.x_rs; m.a_ld = a.D;
+  m.w[0][0] = a.w_up; m.w[0][1] = a.w_gate; m.w_rs[0] = a.w_rs;
+  m.h[0] = static_cast<bf16*>(a.h);
+  const MmPlan p = plan_mm(a.B, a.tok_pad, 2 * (int64_t)a.F, a.D / 64, 1, a.w_fp32 ? kF32Readout : kBf16);
   if (a.w_fp32)
-    launch_both<float>(a, st);
+    launch_mm<true, float>(m, p, st);
   else
-    launch_both<bf16>(a, st);
+    launch_mm<true, bf16>(m, p, st);
+}
+
+void launch_readout_down(const ReadoutMmArgs& a, hipStream_t st) {
+  MmArgs z{};
+  z.B = a.B; z.nseg = 1; z.rows = a.tok_pad; z.rows_pad = a.tok_pad; z.K = a.F; z.N = a.D;
+  z.a[0] = static_cast<const bf16*>(a.h); z.a_rs[0] = (int64_t)a.tok_pad * a.F; z.a_ld = a.F;
+  z.w[0][0] = a.w_down; z.w_rs[0] = a.w_rs;
+  z.zp = a.zp;
+  const MmPlan p = plan_down(a.B, a.T, a.D, a.F, a.w_fp32);
+  if (a.w_fp32)
+    launch_mm<false, float>(z, p, st);
+  else
+    launch_mm<false, bf16>(z, p, st);
 }
 
 }  // namespace uttt
