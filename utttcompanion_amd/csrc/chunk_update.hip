@@ -21,7 +21,9 @@
 //                                       apply clip / momentum / decay / inactive-row select to W
 //                                       and S in one pass (bf16, several token blocks: k_row_scalars
 //                                       first)
-// Steps 1, 2 and the readout half of 3 alone are the frozen readout.
+// Steps 1, 2 and the readout half of 3 alone are the frozen readout (from fp32 W, step 2 in whichever
+// of the two kernels readout_mm_down names; through bf16 W up to 64 tokens, steps 1 and 2 are
+// k_up_gate_lds and k_down_partial_lds).
 #include <algorithm>
 #include <mutex>
 

@@ -19,7 +19,8 @@
 // descriptors of a wave (28 against 24 us at 1 x 333 tokens, d 768, F 2048).  Measured for the
 // whole readout against the 64 x 64-tile kernels it replaced: 4 x 2048 tokens, d 2048, F 5504, bf16
 // copies 1536 -> 561 us (988 TFLOP/s), fp32 masters 2524 -> 683 us; 2 x 333 tokens, d 768, F 2048
-// 39 -> 28 us and 34 -> 33 us; 128 tokens, d 2048, F 5504 52 -> 33 us and 60 -> 44 us.
+// 39 -> 28 us and 34 -> 33 us (there the down product is theirs still, see readout_mm_down); 128 tokens,
+// d 2048, F 5504 52 -> 33 us and 60 -> 44 us.
 #include "readout_mm.h"
 
 #include <algorithm>
