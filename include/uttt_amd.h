@@ -316,6 +316,8 @@ typedef struct {
   int32_t sweep_reverse;
 } uttt_readout_args;
 
+/* Bytes of one such call.  Query each shape: fewer rows or tokens can need more, where the down
+ * product is split further; a workspace too small is refused. */
 size_t uttt_readout_workspace(int64_t batch, int64_t tokens, int64_t d_model, int64_t d_ff, int32_t act_dtype);
 int uttt_swiglu_readout(const uttt_readout_args* args, void* workspace, size_t workspace_bytes,
                         uttt_stream_t stream);

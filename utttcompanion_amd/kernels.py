@@ -961,7 +961,8 @@ def greedy_select(logits: Tensor, banned: Sequence[int] = (), active_limit: Opti
 
 def readout_workspace(x: Tensor, w_up: Tensor) -> Tensor:
     """A workspace for ``swiglu_readout`` of x (B, T, D) through weights shaped like ``w_up``,
-    reusable by every later call with the same or smaller shapes."""
+    reused by every later call that it is large enough for.  A call of fewer rows or tokens can need
+    more, where its down product is split further; ``swiglu_readout`` then allocates its own."""
     bsz, tokens, dim = x.shape
     nbytes = N.load_library().uttt_readout_workspace(bsz, tokens, dim, w_up.shape[-1], _act_code(x.dtype))
     return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
